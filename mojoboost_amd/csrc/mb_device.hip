@@ -599,7 +599,9 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
         // queries the LDS sort holds go to k_lambdarank; larger ones to
         // k_lambdarank_big, which sorts in a global slot per block
         int max_small = 1, max_big = 0;
-        std::vector<int32_t> big;
+        std::vector<int32_t> big, order((size_t)nq);
+        // the small ones by size, largest first (a counting sort)
+        std::vector<int32_t> at(mb::kMaxQueryRows + 2, 0);
         for (int64_t q = 0; q < nq; ++q) {
             const int c = (int)(ds->qstart[q + 1] - ds->qstart[q]);
             if (c > mb::kMaxQueryRows) {
@@ -607,9 +609,23 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
                 max_big = std::max(max_big, c);
             } else {
                 max_small = std::max(max_small, c);
+                ++at[c];
             }
         }
-        int pad = 1;
+        for (int c = mb::kMaxQueryRows, sum = 0; c >= 0; --c) {
+            const int v = at[c];
+            at[c] = sum;
+            sum += v;
+        }
+        for (int64_t q = 0; q < nq; ++q) {
+            const int c = (int)(ds->qstart[q + 1] - ds->qstart[q]);
+            if (c <= mb::kMaxQueryRows) order[(size_t)at[c]++] = (int32_t)q;
+        }
+        s.n_small = (int32_t)(nq - (int64_t)big.size());
+        int32_t *d_order = dalloc<int32_t>(order.size(), run.owned);
+        HIPX(hipMemcpy(d_order, order.data(), order.size() * sizeof(int32_t), hipMemcpyHostToDevice));
+        s.rank_order = d_order;
+        int pad = 8;
         while (pad < max_small) pad <<= 1;
         s.rank_pad = pad;
         if (!big.empty()) {

@@ -324,44 +324,64 @@ __global__ __launch_bounds__(256) void k_objective(DevState s) {
 // :573-600), one block per query, in binary64 as the reference's ranker
 // keeps them. The query's documents are sorted by score in LDS (bitonic,
 // descending, ties by position: the reference's stable order). The pairs
-// (i, j), i below the truncation level, j > i, are then taken one rank i at
-// a time: the block evaluates row i's pairs in parallel, each rank j > i
-// adds its one contribution (it receives the pairs in i order, as in the
-// reference's loop), and two threads add row i's values in j order into the
-// running sum of |lambda| and into rank i's own gradient. Every sum thus has
-// the reference's order and the lambdas its bits. Query LDS: 49 bytes per
-// document of the largest query (rounded up to a power of two).
+// (i, j), i below the truncation level, j > i, are then taken a tile of ranks
+// i at a time. Every sum keeps the reference's order, and so its bits:
+//   - every wave but the first evaluates the next tile's pairs into one of
+//     two LDS buffers;
+//   - rank j adds its tile contributions in i order (column sums);
+//   - meanwhile lanes 0-2 of the first wave walk the tile in (i, j) order:
+//     the running sum of |lambda| and rank i's own lambda and hessian, one
+//     dependent add per pair each, their operands two register blocks ahead.
+// That walk bounds the kernel: a query of 500 documents has 14.5K pairs at
+// truncation 30, about 10 cycles each, so the largest query's walk (~60 us)
+// is its floor, and queries start largest first (rank_order). A pair without
+// a contribution holds -0.0, which no sum here can notice, so the walk has no
+// branch per pair. 120K documents in queries of 1 to 500: 169 us (four waves
+// per SIMD; held to 80 or 64 registers for six or eight: 180, 188), 1534
+// with one rank at a time, a branch and a dependent LDS read per pair and the
+// block waiting at two barriers per rank.
+constexpr int kRankThreads = 512;
+constexpr int kRankEval = kRankThreads - 64;  // pairs of a tile, at most, when it has several ranks
+// LDS of queries padded to `pad` documents (a power of two, at least 8): per
+// document the sort key and position, the gain of its label, its discount and
+// its two sums; two tiles of two values per pair; and two blocks of eight
+// values the walk may read past the last tile.
+__host__ __device__ constexpr int rank_tile_pairs(int pad) { return pad > kRankEval ? pad : kRankEval; }
+__host__ __device__ constexpr size_t rank_lds_for(int pad) {
+    return (size_t)pad * 44 + (size_t)rank_tile_pairs(pad) * 32 + 16 * 8;
+}
+static_assert(rank_lds_for(kMaxQueryRows) + 1024 <= 160 * 1024, "the largest LDS query");
 __device__ __forceinline__ bool rank_before(double ka, int ia, double kb, int ib) {
     return ka > kb || (ka == kb && ia < ib);
 }
 
-__global__ __launch_bounds__(256) void k_lambdarank(DevState s) {
+__global__ __launch_bounds__(kRankThreads) void k_lambdarank(DevState s) {
     extern __shared__ unsigned char rank_lds[];
     __shared__ double s_factor;
-    __shared__ double red_g[4], red_h[4];
+    __shared__ double red_g[kRankThreads / 64], red_h[kRankThreads / 64];
     const Round rd = *s.round;
     if (rd.stopped) return;
     const HyperParams &hp = s.hp;
     if (blockIdx.x == 0 && threadIdx.x == 0) s.cursor[0] = 0;  // root row count
-    const int P = s.rank_pad;
+    const int P = s.rank_pad, cap = rank_tile_pairs(P);
     double *key = (double *)rank_lds;
     double *G = key + P;
     double *H = G + P;
-    double *PL = H + P;
-    double *PH = PL + P;
-    int32_t *idx = (int32_t *)(PH + P);
-    int32_t *lab = idx + P;
-    uint8_t *V = (uint8_t *)(lab + P);
-    const int tid = threadIdx.x, nt = blockDim.x;
+    double *gain = H + P;
+    double *disc = gain + P;
+    double *SG = disc + P;       // two tiles: rank i's own addend of each pair
+    double *SH = SG + 2 * cap;   // and its hessian
+    int32_t *idx = (int32_t *)(SH + 2 * cap + 16);
+    const int tid = threadIdx.x, nt = blockDim.x, lane = lane_id();
     const double sigma = hp.rank_sigma;
     const bool norm = hp.rank_norm != 0;
     const uint64_t bstream = hp.bagging ? bag_stream_of(hp, rd.round) : 0;
     const int64_t bfall = hp.bagging ? bag_fallback_of(s, rd.round) : -1;
     double mg = 0.0, mh = 0.0;
-    for (int q = blockIdx.x; q < s.n_queries; q += gridDim.x) {
+    for (int qi = blockIdx.x; qi < s.n_small; qi += gridDim.x) {
+        const int q = s.rank_order[qi];
         const int64_t a = s.qstart[q];
         const int cnt = (int)(s.qstart[q + 1] - a);
-        if (cnt > kMaxQueryRows) continue;  // k_lambdarank_big's (block-uniform)
         int p2 = 1;
         while (p2 < cnt) p2 <<= 1;
         for (int i = tid; i < p2; i += nt) {
@@ -388,7 +408,8 @@ __global__ __launch_bounds__(256) void k_lambdarank(DevState s) {
                 __syncthreads();
             }
         for (int k = tid; k < cnt; k += nt) {
-            lab[k] = (int)s.labels[a + idx[k]];
+            gain[k] = label_gain((int)s.labels[a + idx[k]]);
+            disc[k] = s.rank_disc[k];
             G[k] = 0.0;
             H[k] = 0.0;
         }
@@ -396,55 +417,103 @@ __global__ __launch_bounds__(256) void k_lambdarank(DevState s) {
         const double best = key[0], worst = key[cnt - 1];
         const double inv = s.inv_max_dcg[q];
         const int top = cnt - 1 < hp.rank_trunc ? cnt - 1 : hp.rank_trunc;
-        double sum = 0.0;  // thread 0's running sum of |lambda| (ranking.mojo:565)
-        for (int i = 0; i < top; ++i) {
-            const int li = lab[i];
-            const double si = key[i];
-            for (int j = i + 1 + tid; j < cnt; j += nt) {
-                const int lj = lab[j];
-                double pl = 0.0, ph = 0.0;
-                uint8_t v = 0;
-                if (li != lj) {
-                    const bool ih = li > lj;  // rank i holds the more relevant document
-                    const int hr = ih ? i : j, lr = ih ? j : i;
-                    const double delta = ih ? si - key[j] : key[j] - si;
-                    const double gap = label_gain(ih ? li : lj) - label_gain(ih ? lj : li);
-                    const double paired = fabs(s.rank_disc[hr] - s.rank_disc[lr]);
-                    double dn = gap * paired * inv;
+        // a rank's row of a tile: its pairs at j, -0.0 at every j <= i and
+        // from cnt to the next multiple of eight
+        const int row = (cnt + 7) & ~7;
+        const int tile = kRankEval / row > 1 ? kRankEval / row : 1;  // ranks of a tile: tile x row <= cap
+        auto evaluate = [&](int i0, int b) {
+            const int rows = top - i0 < tile ? top - i0 : tile;
+            double *sg = SG + b * cap, *sh = SH + b * cap;
+            for (int e = tid - 64; e < rows * row; e += kRankEval) {
+                const int ii = e / row, j = e - ii * row, i = i0 + ii;
+                double vg = -0.0, vh = -0.0;
+                const double gi = gain[i], gj = j < cnt ? gain[j] : gi;
+                if (j > i && gi != gj) {  // labels differ as their gains do
+                    const bool ih = gi > gj;  // rank i holds the more relevant document
+                    const double ki = key[i], kj = key[j];
+                    const double delta = ih ? ki - kj : kj - ki;
+                    const double paired = fabs(disc[i] - disc[j]);
+                    double dn = (ih ? gi - gj : gj - gi) * paired * inv;
                     if (norm && best != worst) dn /= 0.01 + fabs(delta);
                     double p = pair_sigmoid(delta, sigma);
                     double phh = p * (1.0 - p);
-                    p *= -sigma * dn;
+                    p *= -sigma * dn;  // the pair's lambda, never above zero
                     phh *= sigma * sigma * dn;
-                    pl = p;
-                    ph = phh;
-                    v = ih ? 3 : 1;
-                    G[j] = ih ? G[j] - p : G[j] + p;
-                    H[j] = H[j] + phh;
+                    vg = ih ? p : -p;
+                    vh = phh;
                 }
-                PL[j] = pl;
-                PH[j] = ph;
-                V[j] = v;
+                sg[e] = vg;
+                sh[e] = vh;
+            }
+        };
+        double sum = 0.0;  // lane 0: half the running sum of |lambda| (ranking.mojo:565)
+        if (tid >= 64) evaluate(0, 0);
+        __syncthreads();
+        for (int i0 = 0, b = 0; i0 < top; i0 += tile, b ^= 1) {
+            const int rows = top - i0 < tile ? top - i0 : tile;
+            const double *sg = SG + b * cap, *sh = SH + b * cap;
+            for (int j = i0 + 1 + tid; j < cnt; j += nt) {
+                double g = G[j], h = H[j];
+#pragma unroll 4
+                for (int ii = 0; ii < rows; ++ii) {
+                    g -= sg[ii * row + j];
+                    h += sh[ii * row + j];
+                }
+                G[j] = g;
+                H[j] = h;
             }
             __syncthreads();
-            if (tid == 0) {
-                for (int j = i + 1; j < cnt; ++j)
-                    if (V[j]) sum -= 2.0 * PL[j];
-            } else if (tid == 64) {
-                double g = G[i], h = H[i];
-                for (int j = i + 1; j < cnt; ++j) {
-                    const uint8_t v = V[j];
-                    if (!v) continue;
-                    g = (v & 2) ? g + PL[j] : g - PL[j];
-                    h = h + PH[j];
+            if (tid >= 64) {
+                evaluate(i0 + tile, b ^ 1);
+            } else if (lane < 3) {
+                // lane 0: |lambda| (the addend up to its sign; the sum is
+                // doubled at the end, which is exact), lane 1: the lambda,
+                // lane 2: the hessian
+                __builtin_amdgcn_s_setprio(3);
+                const unsigned long long keep = lane == 0 ? ~(1ULL << 63) : ~0ULL;
+                const double *src = lane == 2 ? sh : sg;
+                for (int ii = 0; ii < rows; ++ii, src += row) {
+                    const int i = i0 + ii;
+                    double run = lane == 0 ? sum : lane == 1 ? G[i] : H[i];
+                    double2 x0[4], x1[4], x2[4];
+                    auto load = [&](double2 *x, int at) {
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) x[u] = ((const double2 *)(src + at))[u];
+                    };
+                    auto one = [&](double v) {
+                        run += __longlong_as_double((long long)((unsigned long long)__double_as_longlong(v) & keep));
+                    };
+                    auto add = [&](const double2 *x) {
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            one(x[u].x);
+                            one(x[u].y);
+                        }
+                    };
+                    int j = (i + 1) & ~7;
+                    load(x0, j);
+                    load(x1, j + 8);
+                    for (;;) {
+                        load(x2, j + 16);
+                        add(x0);
+                        if ((j += 8) >= row) break;
+                        load(x0, j + 16);
+                        add(x1);
+                        if ((j += 8) >= row) break;
+                        load(x1, j + 16);
+                        add(x2);
+                        if ((j += 8) >= row) break;
+                    }
+                    if (lane == 0) sum = run;
+                    else (lane == 1 ? G : H)[i] = run;
                 }
-                G[i] = g;
-                H[i] = h;
+                __builtin_amdgcn_s_setprio(0);
             }
             __syncthreads();
         }
         // the query's normalizer log2(1 + S) / S (ranking.mojo:567-570); 0
         // marks "not applied"
+        sum *= 2.0;
         if (tid == 0) s_factor = (norm && sum > 0.0) ? ref_log2(1.0 + sum) / sum : 0.0;
         __syncthreads();
         const double factor = s_factor;
@@ -488,9 +557,13 @@ __global__ __launch_bounds__(256) void k_lambdarank(DevState s) {
             mg = fmax(mg, red_g[i]);
             mh = fmax(mh, red_h[i]);
         }
-        // non-negative doubles order like their bit patterns
-        atomicMax(&s.stats64[rd.parity * 2 + 0], (unsigned long long)__double_as_longlong(mg));
-        atomicMax(&s.stats64[rd.parity * 2 + 1], (unsigned long long)__double_as_longlong(mh));
+        // non-negative doubles order like their bit patterns; a maximum only
+        // grows, so a block at or below what it reads has nothing to add
+        const unsigned long long bg = (unsigned long long)__double_as_longlong(mg);
+        const unsigned long long bh = (unsigned long long)__double_as_longlong(mh);
+        unsigned long long *st = &s.stats64[rd.parity * 2];
+        if (bg > load_agent(&st[0])) atomicMax(&st[0], bg);
+        if (bh > load_agent(&st[1])) atomicMax(&st[1], bh);
     }
 }
 
@@ -5672,11 +5745,13 @@ __global__ void k_exp_sigmoid(const double *x, double *e, double *sg, int64_t n)
 }
 
 // ------------------------------------------------------------------ launch
-size_t rank_lds_bytes(const DevState &s) { return (size_t)s.rank_pad * 49; }
+size_t rank_lds_bytes(const DevState &s) { return rank_lds_for(s.rank_pad); }
 hipError_t launch_objective(const DevState &s, int grid, hipStream_t st) {
     if (s.hp.objective == kObjLambdarank) {
-        const int g = s.n_queries < 4 * grid ? s.n_queries : 4 * grid;
-        hipLaunchKernelGGL(k_lambdarank, dim3(g > 0 ? g : 1), dim3(256), rank_lds_bytes(s), st, s);
+        // a block per query, as many as may be in flight; the next queries
+        // of rank_order go to the blocks that end first
+        const int g = s.n_small > 1 ? s.n_small : 1;
+        hipLaunchKernelGGL(k_lambdarank, dim3(g), dim3(kRankThreads), rank_lds_bytes(s), st, s);
         if (s.n_big > 0) {
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;

@@ -311,7 +311,9 @@ struct DevState {
     const double *inv_max_dcg;      // per query: 1 / maxDCG at the truncation level (0: none)
     const double *rank_disc;        // 1 / log2(rank + 2) for ranks below the largest query
     int32_t n_queries;
-    int32_t rank_pad;               // largest query of at most kMaxQueryRows rows, rounded up to a power of two
+    int32_t n_small;                // queries of at most kMaxQueryRows rows
+    const int32_t *rank_order;      // n_small: those queries, largest first
+    int32_t rank_pad;               // largest query of at most kMaxQueryRows rows, rounded up to a power of two (at least 8)
     // queries of more than kMaxQueryRows rows (k_lambdarank_big): their
     // indices, and per block slot the query's keys, G, H (binary64) and
     // positions, labels (int32), each rank_big_pad long
