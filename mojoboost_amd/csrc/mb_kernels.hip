@@ -870,6 +870,49 @@ __device__ __forceinline__ int32_t quant_value(const QCtx &c, float v, bool w, i
                            (isg ? c.gs : c.hs) + (uint64_t)r);
 }
 
+// The bag's rows as the root list, a tile of kBagTile consecutive rows per
+// block pass: the draws' ballots give each wave its place in the tile and one
+// atomic per tile its place in the list (an atomic per wave on the one
+// address, 15.6K of them for 1M rows, serialized in the L2: k_quantize 194 us
+// there, 14 us with the tiles). The order of the tiles does not matter (the
+// histograms' integer sums have none, the binary64 ones no fixed one).
+constexpr int kBagRows = 16;  // rows of a thread of a tile
+constexpr int kBagTile = 256 * kBagRows;
+__device__ __forceinline__ void list_bag(const DevState &s, uint64_t bstream, int64_t bfall) {
+    __shared__ int wave_n[4];
+    __shared__ long long s_base;
+    const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
+    const unsigned long long below = (1ULL << lane) - 1ULL;
+    for (int64_t r0 = (int64_t)blockIdx.x * kBagTile; r0 < s.n; r0 += (int64_t)gridDim.x * kBagTile) {
+        uint32_t take = 0;
+        int mine = 0;  // the wave's rows (wave-uniform)
+#pragma unroll
+        for (int u = 0; u < kBagRows; ++u) {
+            const int64_t r = r0 + u * 256 + tid;
+            const bool t = r < s.n && in_bag(s, bstream, bfall, r);
+            take |= (t ? 1u : 0u) << u;
+            mine += (int)__popcll(__ballot(t));
+        }
+        if (lane == 0) wave_n[w] = mine;
+        __syncthreads();
+        if (tid == 0) {
+            const int all = wave_n[0] + wave_n[1] + wave_n[2] + wave_n[3];
+            s_base = all ? (long long)atomicAdd((unsigned long long *)&s.cursor[0], (unsigned long long)all) : 0;
+        }
+        __syncthreads();
+        long long at = s_base;
+        for (int i = 0; i < w; ++i) at += wave_n[i];
+#pragma unroll
+        for (int u = 0; u < kBagRows; ++u) {
+            const bool t = (take >> u) & 1u;
+            const unsigned long long m = __ballot(t);
+            if (t) s.rows0[at + __popcll(m & below)] = (int32_t)(r0 + u * 256 + tid);
+            at += __popcll(m);
+        }
+        __syncthreads();  // the counts are the next tile's
+    }
+}
+
 // write_pairs = 0: the max-abs int8 pairs are left to the root build
 // (k_hist quantizes the rows it reads, k_hist<.., kQuant>); the scales and
 // the root row list are still published here.
@@ -910,10 +953,12 @@ __device__ __forceinline__ void quantize_body(const DevState &s, int write_pairs
     if (!(hp.quantized && write_pairs) && !copy_sample && !(hp.bagging && !gs_on)) return;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     const int rec = s.rec_bytes;
-    for (int64_t r0 = (int64_t)blockIdx.x * blockDim.x; r0 < s.n; r0 += stride) {
+    const bool pairs = hp.quantized && write_pairs;
+    const int64_t per_row = pairs || copy_sample ? s.n : 0;
+    for (int64_t r0 = (int64_t)blockIdx.x * blockDim.x; r0 < per_row; r0 += stride) {
         const int64_t r = r0 + threadIdx.x;
         const bool valid = r < s.n;
-        if (valid && hp.quantized && write_pairs) {
+        if (valid && pairs) {
             int32_t qg, qh;
             quant_row(s, c, r, qg, qh);
             if (hp.stage16) {
@@ -945,24 +990,11 @@ __device__ __forceinline__ void quantize_body(const DevState &s, int write_pairs
                     *hw = *hw | 0x80000000u;
                 }
             }
-        } else if (!hp.bagging) {
-            // every row in order: the root build and the root's partition
-            // compute the ids, no list is written
-        } else {
-            // Sampled rows appended with one atomic per wave; their order in
-            // the root range does not matter (integer histograms).
-            bool take = valid && in_bag(s, bstream, bfall, r);
-            unsigned long long m = __ballot(take);
-            int cnt = __popcll(m);
-            long long base = 0;
-            if (lane_id() == 0 && cnt) base = atomicAdd((unsigned long long *)&s.cursor[0], (unsigned long long)cnt);
-            base = __shfl(base, 0, 64);
-            if (take) {
-                int rank = __popcll(m & ((1ULL << lane_id()) - 1ULL));
-                s.rows0[base + rank] = (int32_t)r;
-            }
         }
     }
+    // (without a sample every row in order: the root build and the root's
+    // partition compute the ids, no list is written)
+    if (hp.bagging && !gs_on) list_bag(s, bstream, bfall);
 }
 
 __global__ __launch_bounds__(256) void k_quantize(DevState s, int write_pairs) { quantize_body(s, write_pairs); }
