@@ -18,6 +18,8 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <memory>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -55,6 +57,121 @@ T *dalloc(size_t count, std::vector<void *> &owned) {
     HIPX(hipMalloc(&p, bytes));
     owned.push_back(p);
     return (T *)p;
+}
+
+// Device memory of the library's calls on a dataset. A call places its
+// buffers in slabs (Arena) instead of allocating each one, and leaves the
+// slabs to the dataset's next call: a training places some 100 buffers, and
+// allocating and freeing them took 0.5 ms on a small table and 6 ms for ten
+// classes on 300K x 50. Idle slabs belong to their dataset, are freed with
+// it, total at most kIdleMost over the process, and are all freed when an
+// allocation fails. Calls on one dataset at a time share nothing: a call takes
+// every idle slab of its dataset, a second one beside it finds none.
+struct Slab {
+    uint8_t *p = nullptr;
+    size_t size = 0;
+    const void *owner = nullptr;
+};
+
+class SlabPool {
+public:
+    std::vector<Slab> take(const void *owner) {
+        std::lock_guard<std::mutex> lock(mu_);
+        std::vector<Slab> mine;
+        for (size_t i = idle_.size(); i-- > 0;)
+            if (idle_[i].owner == owner) {
+                mine.insert(mine.begin(), idle_[i]);
+                bytes_ -= idle_[i].size;
+                idle_.erase(idle_.begin() + (ptrdiff_t)i);
+            }
+        return mine;
+    }
+    // the slabs must be idle on the device
+    void give(std::vector<Slab> &slabs) {
+        std::lock_guard<std::mutex> lock(mu_);
+        for (const Slab &s : slabs) {
+            if (s.owner && bytes_ + s.size <= kIdleMost) {
+                idle_.push_back(s);
+                bytes_ += s.size;
+            } else {
+                (void)hipFree(s.p);
+            }
+        }
+        slabs.clear();
+    }
+    // an owner's idle slabs, or every one
+    void drop(const void *owner, bool all = false) {
+        std::lock_guard<std::mutex> lock(mu_);
+        for (size_t i = idle_.size(); i-- > 0;)
+            if (all || idle_[i].owner == owner) {
+                (void)hipFree(idle_[i].p);
+                bytes_ -= idle_[i].size;
+                idle_.erase(idle_.begin() + (ptrdiff_t)i);
+            }
+    }
+
+private:
+    static constexpr size_t kIdleMost = (size_t)4 << 30;
+    std::mutex mu_;
+    std::vector<Slab> idle_;
+    size_t bytes_ = 0;
+};
+
+// Never destroyed: the HIP runtime may be gone when static objects are.
+SlabPool &slab_pool() {
+    static SlabPool *pool = new SlabPool();
+    return *pool;
+}
+
+// The buffers of one call, in the slabs its dataset's last call left and in
+// new ones.
+class Arena {
+public:
+    explicit Arena(const void *owner) : owner_(owner) {
+        if (owner) slabs_ = slab_pool().take(owner);
+    }
+    Arena(const Arena &) = delete;
+    Arena &operator=(const Arena &) = delete;
+    ~Arena() {
+        // as the frees did, wait for whatever still uses the buffers
+        if (!slabs_.empty()) (void)hipDeviceSynchronize();
+        slab_pool().give(slabs_);
+    }
+    void *place(size_t bytes) {
+        bytes = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
+        // first fit over the slabs' free ends
+        used_.resize(slabs_.size(), 0);
+        for (size_t i = 0; i < slabs_.size(); ++i)
+            if (slabs_[i].size - used_[i] >= bytes) {
+                void *at = slabs_[i].p + used_[i];
+                used_[i] += bytes;
+                return at;
+            }
+        Slab s;
+        s.owner = owner_;
+        s.size = std::max(bytes, kSlab);
+        hipError_t e = hipMalloc((void **)&s.p, s.size);
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            slab_pool().drop(nullptr, true);
+            s.size = bytes;
+            HIPX(hipMalloc((void **)&s.p, s.size));
+        }
+        slabs_.push_back(s);
+        used_.push_back(bytes);
+        return s.p;
+    }
+
+private:
+    static constexpr size_t kSlab = (size_t)32 << 20;
+    const void *owner_;
+    std::vector<Slab> slabs_;
+    std::vector<size_t> used_;
+};
+
+template <class T>
+T *dalloc(size_t count, Arena &arena) {
+    return (T *)arena.place(count * sizeof(T));
 }
 
 int device_count_gfx950() {
@@ -134,11 +251,48 @@ struct mbh_dataset {
     int max_query = 0;
     std::vector<void *> owned;
     ~mbh_dataset() {
+        slab_pool().drop(this);
         for (void *p : owned) (void)hipFree(p);
     }
 };
 
 constexpr int kNumStats = 22;
+
+// A fit's raw scores on the host: pinned from kPinBytes on (the copy from the
+// device then runs at the link's rate, 84 MB in 1.6 ms against 5 into
+// pageable memory after 14 of zeroing a vector), else ordinary memory,
+// not zeroed first.
+struct HostScores {
+    double *p = nullptr;
+    size_t n = 0;
+    bool pinned = false;
+    void reserve(size_t count) {
+        release();
+        if (count * sizeof(double) >= kPinBytes) {
+            pinned = hipHostMalloc((void **)&p, count * sizeof(double), hipHostMallocDefault) == hipSuccess;
+            if (!pinned) {
+                (void)hipGetLastError();
+                p = nullptr;
+            }
+        }
+        if (!p) p = new double[count > 0 ? count : 1];
+        n = count;
+    }
+    void release() {
+        if (pinned) (void)hipHostFree(p);
+        else delete[] p;
+        p = nullptr;
+        n = 0;
+        pinned = false;
+    }
+    HostScores() = default;
+    HostScores(const HostScores &) = delete;
+    HostScores &operator=(const HostScores &) = delete;
+    ~HostScores() { release(); }
+
+private:
+    static constexpr size_t kPinBytes = (size_t)1 << 20;
+};
 
 struct mbh_fit {
     int num_class = 1;
@@ -150,7 +304,7 @@ struct mbh_fit {
     std::vector<int32_t> feature, threshold, left, right, default_left, missing_bin;
     std::vector<double> value, gain, count;
     std::vector<uint64_t> cat_bits;  // 4 words per node
-    std::vector<double> train_raw;
+    HostScores train_raw;
     double stats[kNumStats] = {0};
     // time_histograms runs: per expansion launch, (tree, iteration, rows
     // partitioned, rows accumulated, partition ms, accumulation ms)
@@ -160,10 +314,8 @@ struct mbh_fit {
 namespace {
 
 struct Run {
-    std::vector<void *> owned;
-    ~Run() {
-        for (void *p : owned) (void)hipFree(p);
-    }
+    Arena arena;
+    explicit Run(const mbh_dataset *ds) : arena(ds) {}
 };
 
 struct PinnedFlags {
@@ -413,15 +565,15 @@ void configure_hist(mb::DevState &s, const mbh_dataset *ds, int B, int kind, Run
                                             s.pb_grid);
     const size_t cells = (size_t)parts * ds->F * s.part_stride;
     if (quantized) {
-        s.part = dalloc<unsigned long long>(cells, run.owned);
-        if (kind == mb::kAccWide) s.part_c = dalloc<uint32_t>(cells, run.owned);
+        s.part = dalloc<unsigned long long>(cells, run.arena);
+        if (kind == mb::kAccWide) s.part_c = dalloc<uint32_t>(cells, run.arena);
     } else {
-        s.fpart_g = dalloc<double>(cells, run.owned);
-        s.fpart_h = dalloc<double>(cells, run.owned);
-        s.fpart_c = dalloc<uint32_t>(cells, run.owned);
+        s.fpart_g = dalloc<double>(cells, run.arena);
+        s.fpart_h = dalloc<double>(cells, run.arena);
+        s.fpart_c = dalloc<uint32_t>(cells, run.arena);
     }
-    s.part_items = dalloc<mb::PartItem>(s.kmax, run.owned);
-    s.acc_items = dalloc<mb::AccItem>(s.kmax, run.owned);
+    s.part_items = dalloc<mb::PartItem>(s.kmax, run.arena);
+    s.acc_items = dalloc<mb::AccItem>(s.kmax, run.arena);
 }
 
 double base_score_for(const mbh_dataset *ds, int objective) {
@@ -491,65 +643,65 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
     s.tile_f = ds->tile_f;
     s.n_tiles = ds->n_tiles;
     s.lds_stride = ds->lds_stride;
-    s.raw = dalloc<double>((size_t)ds->n * K, run.owned);
-    s.prob = K > 1 ? dalloc<double>((size_t)ds->n * K, run.owned) : nullptr;
-    s.grad = dalloc<float>(ds->n, run.owned);
-    s.hess = dalloc<float>(ds->n, run.owned);
-    s.stats = dalloc<uint32_t>(4 * mb::kStatSlots, run.owned);
-    s.round = dalloc<mb::Round>(1, run.owned);
-    s.rows0 = dalloc<int32_t>(ds->n, run.owned);
-    s.rows1 = dalloc<int32_t>(ds->n, run.owned);
+    s.raw = dalloc<double>((size_t)ds->n * K, run.arena);
+    s.prob = K > 1 ? dalloc<double>((size_t)ds->n * K, run.arena) : nullptr;
+    s.grad = dalloc<float>(ds->n, run.arena);
+    s.hess = dalloc<float>(ds->n, run.arena);
+    s.stats = dalloc<uint32_t>(4 * mb::kStatSlots, run.arena);
+    s.round = dalloc<mb::Round>(1, run.arena);
+    s.rows0 = dalloc<int32_t>(ds->n, run.arena);
+    s.rows1 = dalloc<int32_t>(ds->n, run.arena);
     const int max_exp = std::min(4 * L - 1, 2047);
     s.max_exp = max_exp;
     s.e_cap = 1 + 2 * max_exp;
-    if (quantized) s.hist = dalloc<int32_t>((size_t)(1 + max_exp) * F * ds->nb * 3, run.owned);
-    else s.histf = dalloc<mb::HistF>((size_t)(1 + max_exp) * F * ds->nb, run.owned);
+    if (quantized) s.hist = dalloc<int32_t>((size_t)(1 + max_exp) * F * ds->nb * 3, run.arena);
+    else s.histf = dalloc<mb::HistF>((size_t)(1 + max_exp) * F * ds->nb, run.arena);
     configure_hist(s, ds, quantized ? p->num_grad_quant_bins : 4, kind, run);
     if (wide) {
-        if (!stage16) s.gq = dalloc<int32_t>(2 * (size_t)ds->n, run.owned);
-        s.magpart = dalloc<float>(2 * 256, run.owned);
-        s.stage16_over = dalloc<unsigned long long>(2, run.owned);
+        if (!stage16) s.gq = dalloc<int32_t>(2 * (size_t)ds->n, run.arena);
+        s.magpart = dalloc<float>(2 * 256, run.arena);
+        s.stage16_over = dalloc<unsigned long long>(2, run.arena);
         HIPX(hipMemset(s.stage16_over, 0, 2 * sizeof(unsigned long long)));
     }
-    s.enodes = dalloc<mb::ENode>(s.e_cap, run.owned);
-    s.items = dalloc<mb::Item>(s.kmax, run.owned);
-    s.batch = dalloc<mb::Batch>(1, run.owned);
-    s.grow = dalloc<mb::Grow>(1, run.owned);
-    s.slot_e = dalloc<int32_t>(L, run.owned);
-    s.slot_fid = dalloc<int32_t>(L, run.owned);
-    s.scan = dalloc<mb::ScanResult>((size_t)s.kmax * 2 * F, run.owned);
-    s.scan_gain = dalloc<double>((size_t)s.kmax * 2 * F, run.owned);
-    s.pair_gain = dalloc<double>((size_t)s.kmax * 2, run.owned);
-    s.pair_feat = dalloc<int32_t>((size_t)s.kmax * 2, run.owned);
-    s.e_gain = dalloc<double>(s.e_cap, run.owned);
-    s.e_left = dalloc<int32_t>(s.e_cap, run.owned);
-    s.e_rows = dalloc<int32_t>(s.e_cap, run.owned);
-    s.e_parent = dalloc<int32_t>(s.e_cap, run.owned);
-    s.cursor = dalloc<int64_t>(2 + 2 * (size_t)s.kmax, run.owned);
-    s.error = dalloc<int32_t>(1, run.owned);
-    s.t_feature = dalloc<int32_t>(max_nodes, run.owned);
-    s.t_threshold = dalloc<int32_t>(max_nodes, run.owned);
-    s.t_left = dalloc<int32_t>(max_nodes, run.owned);
-    s.t_right = dalloc<int32_t>(max_nodes, run.owned);
-    s.t_default_left = dalloc<int32_t>(max_nodes, run.owned);
-    s.t_missing_bin = dalloc<int32_t>(max_nodes, run.owned);
-    s.t_value = dalloc<double>(max_nodes, run.owned);
-    s.t_gain = dalloc<double>(max_nodes, run.owned);
-    s.t_count = dalloc<double>(max_nodes, run.owned);
-    s.t_meta = dalloc<int32_t>(2, run.owned);
-    s.arc_int = dalloc<int32_t>((size_t)T * (6 * max_nodes + 2), run.owned);
-    s.arc_dbl = dalloc<double>((size_t)T * 3 * max_nodes, run.owned);
-    s.arc_aux = dalloc<int64_t>((size_t)T * 4, run.owned);
+    s.enodes = dalloc<mb::ENode>(s.e_cap, run.arena);
+    s.items = dalloc<mb::Item>(s.kmax, run.arena);
+    s.batch = dalloc<mb::Batch>(1, run.arena);
+    s.grow = dalloc<mb::Grow>(1, run.arena);
+    s.slot_e = dalloc<int32_t>(L, run.arena);
+    s.slot_fid = dalloc<int32_t>(L, run.arena);
+    s.scan = dalloc<mb::ScanResult>((size_t)s.kmax * 2 * F, run.arena);
+    s.scan_gain = dalloc<double>((size_t)s.kmax * 2 * F, run.arena);
+    s.pair_gain = dalloc<double>((size_t)s.kmax * 2, run.arena);
+    s.pair_feat = dalloc<int32_t>((size_t)s.kmax * 2, run.arena);
+    s.e_gain = dalloc<double>(s.e_cap, run.arena);
+    s.e_left = dalloc<int32_t>(s.e_cap, run.arena);
+    s.e_rows = dalloc<int32_t>(s.e_cap, run.arena);
+    s.e_parent = dalloc<int32_t>(s.e_cap, run.arena);
+    s.cursor = dalloc<int64_t>(2 + 2 * (size_t)s.kmax, run.arena);
+    s.error = dalloc<int32_t>(1, run.arena);
+    s.t_feature = dalloc<int32_t>(max_nodes, run.arena);
+    s.t_threshold = dalloc<int32_t>(max_nodes, run.arena);
+    s.t_left = dalloc<int32_t>(max_nodes, run.arena);
+    s.t_right = dalloc<int32_t>(max_nodes, run.arena);
+    s.t_default_left = dalloc<int32_t>(max_nodes, run.arena);
+    s.t_missing_bin = dalloc<int32_t>(max_nodes, run.arena);
+    s.t_value = dalloc<double>(max_nodes, run.arena);
+    s.t_gain = dalloc<double>(max_nodes, run.arena);
+    s.t_count = dalloc<double>(max_nodes, run.arena);
+    s.t_meta = dalloc<int32_t>(2, run.arena);
+    s.arc_int = dalloc<int32_t>((size_t)T * (6 * max_nodes + 2), run.arena);
+    s.arc_dbl = dalloc<double>((size_t)T * 3 * max_nodes, run.arena);
+    s.arc_aux = dalloc<int64_t>((size_t)T * 4, run.arena);
     if (ds->any_cat) {
-        s.scan_cat = dalloc<unsigned long long>((size_t)s.kmax * 2 * F * 4, run.owned);
-        s.e_cat = dalloc<unsigned long long>((size_t)s.e_cap * 4, run.owned);
-        s.t_cat = dalloc<unsigned long long>((size_t)max_nodes * 4, run.owned);
-        s.arc_cat = dalloc<unsigned long long>((size_t)T * max_nodes * 4, run.owned);
+        s.scan_cat = dalloc<unsigned long long>((size_t)s.kmax * 2 * F * 4, run.arena);
+        s.e_cat = dalloc<unsigned long long>((size_t)s.e_cap * 4, run.arena);
+        s.t_cat = dalloc<unsigned long long>((size_t)max_nodes * 4, run.arena);
+        s.arc_cat = dalloc<unsigned long long>((size_t)T * max_nodes * 4, run.arena);
         HIPX(hipMemset(s.t_cat, 0, (size_t)max_nodes * 4 * sizeof(unsigned long long)));
         HIPX(hipMemset(s.arc_cat, 0, (size_t)T * max_nodes * 4 * sizeof(unsigned long long)));
     }
     s.max_nodes = max_nodes;
-    uint8_t *fmask = dalloc<uint8_t>((size_t)T * F, run.owned);
+    uint8_t *fmask = dalloc<uint8_t>((size_t)T * F, run.arena);
     s.feature_mask = fmask;
     mb::HyperParams &hp = s.hp;
     hp.objective = p->objective;
@@ -572,9 +724,9 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
         hp.rank_trunc = p->lambdarank_truncation_level;
         hp.rank_norm = p->lambdarank_norm ? 1 : 0;
         hp.rank_sigma = p->lambdarank_sigmoid;
-        s.grad64 = dalloc<double>(ds->n, run.owned);
-        s.hess64 = dalloc<double>(ds->n, run.owned);
-        s.stats64 = dalloc<unsigned long long>(4, run.owned);
+        s.grad64 = dalloc<double>(ds->n, run.arena);
+        s.hess64 = dalloc<double>(ds->n, run.arena);
+        s.stats64 = dalloc<unsigned long long>(4, run.arena);
         HIPX(hipMemset(s.stats64, 0, 4 * sizeof(unsigned long long)));
         const int64_t nq = (int64_t)ds->qstart.size() - 1;
         std::vector<double> disc(ds->max_query), inv(nq);
@@ -588,8 +740,8 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
             for (int64_t j = 0; j < m; ++j) md += mb::label_gain(g[j]) * disc[j];
             inv[q] = md > 0.0 ? 1.0 / md : 0.0;
         }
-        double *d_disc = dalloc<double>(std::max(1, ds->max_query), run.owned);
-        double *d_inv = dalloc<double>(nq, run.owned);
+        double *d_disc = dalloc<double>(std::max(1, ds->max_query), run.arena);
+        double *d_inv = dalloc<double>(nq, run.arena);
         HIPX(hipMemcpy(d_disc, disc.data(), disc.size() * sizeof(double), hipMemcpyHostToDevice));
         HIPX(hipMemcpy(d_inv, inv.data(), inv.size() * sizeof(double), hipMemcpyHostToDevice));
         s.rank_disc = d_disc;
@@ -622,7 +774,7 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
             if (c <= mb::kMaxQueryRows) order[(size_t)at[c]++] = (int32_t)q;
         }
         s.n_small = (int32_t)(nq - (int64_t)big.size());
-        int32_t *d_order = dalloc<int32_t>(order.size(), run.owned);
+        int32_t *d_order = dalloc<int32_t>(order.size(), run.arena);
         HIPX(hipMemcpy(d_order, order.data(), order.size() * sizeof(int32_t), hipMemcpyHostToDevice));
         s.rank_order = d_order;
         int pad = 8;
@@ -637,9 +789,9 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
             s.n_big = (int32_t)big.size();
             s.rank_big_pad = bp;
             s.rank_big_slots = slots;
-            s.rank_scratch = dalloc<double>((size_t)slots * 3 * bp, run.owned);
-            s.rank_scratch_i = dalloc<int32_t>((size_t)slots * 2 * bp, run.owned);
-            int32_t *d_big = dalloc<int32_t>(big.size(), run.owned);
+            s.rank_scratch = dalloc<double>((size_t)slots * 3 * bp, run.arena);
+            s.rank_scratch_i = dalloc<int32_t>((size_t)slots * 2 * bp, run.arena);
+            int32_t *d_big = dalloc<int32_t>(big.size(), run.arena);
             HIPX(hipMemcpy(d_big, big.data(), big.size() * sizeof(int32_t), hipMemcpyHostToDevice));
             s.rank_big = d_big;
         }
@@ -657,32 +809,32 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
     hp.goss_exact = p->goss_exact_walk ? 1 : 0;
     if (hp.goss) {
         s.goss_nblk = (int32_t)((ds->n + 1023) / 1024);
-        s.gst = dalloc<mb::GossState>(1, run.owned);
-        s.goss_hist = dalloc<uint32_t>(8 * mb::kGossHistSlots * 256, run.owned);
-        s.goss_sel = dalloc<unsigned long long>(16, run.owned);
-        s.goss_cand = dalloc<unsigned long long>(ds->n, run.owned);
-        s.goss_ccnt = dalloc<int32_t>(mb::kGossDigitBlocks, run.owned);
+        s.gst = dalloc<mb::GossState>(1, run.arena);
+        s.goss_hist = dalloc<uint32_t>(8 * mb::kGossHistSlots * 256, run.arena);
+        s.goss_sel = dalloc<unsigned long long>(16, run.arena);
+        s.goss_cand = dalloc<unsigned long long>(ds->n, run.arena);
+        s.goss_ccnt = dalloc<int32_t>(mb::kGossDigitBlocks, run.arena);
         // padded to whole count tiles; the pad holds INT_MIN (never kept) and
         // no kernel writes it
         const int64_t padded = (ds->n + mb::kGossTileRows - 1) / mb::kGossTileRows * mb::kGossTileRows;
-        s.goss_kappa = dalloc<int32_t>(padded, run.owned);
+        s.goss_kappa = dalloc<int32_t>(padded, run.arena);
         if (padded > ds->n) {
             std::vector<int32_t> pad(padded - ds->n, INT32_MIN);
             HIPX(hipMemcpy(s.goss_kappa + ds->n, pad.data(), pad.size() * sizeof(int32_t), hipMemcpyHostToDevice));
         }
-        s.goss_mask = dalloc<unsigned long long>((ds->n + 63) / 64, run.owned);
-        s.goss_topmask = dalloc<unsigned long long>((ds->n + 63) / 64, run.owned);
-        s.goss_blk = dalloc<int32_t>(s.goss_nblk, run.owned);
-        s.goss_blk_u = dalloc<int32_t>(s.goss_nblk, run.owned);
-        s.goss_ukappa = dalloc<int32_t>(padded, run.owned);  // whole count tiles
-        s.goss_urow = dalloc<int32_t>(ds->n, run.owned);
-        s.goss_umask = dalloc<unsigned long long>((ds->n + 63) / 64, run.owned);
-        s.goss_other = dalloc<uint8_t>(ds->n, run.owned);
+        s.goss_mask = dalloc<unsigned long long>((ds->n + 63) / 64, run.arena);
+        s.goss_topmask = dalloc<unsigned long long>((ds->n + 63) / 64, run.arena);
+        s.goss_blk = dalloc<int32_t>(s.goss_nblk, run.arena);
+        s.goss_blk_u = dalloc<int32_t>(s.goss_nblk, run.arena);
+        s.goss_ukappa = dalloc<int32_t>(padded, run.arena);  // whole count tiles
+        s.goss_urow = dalloc<int32_t>(ds->n, run.arena);
+        s.goss_umask = dalloc<unsigned long long>((ds->n + 63) / 64, run.arena);
+        s.goss_other = dalloc<uint8_t>(ds->n, run.arena);
         HIPX(hipMemset(s.goss_other, 0, ds->n));
-        s.goss_rows = dalloc<int32_t>(ds->n, run.owned);
-        s.goss_max = dalloc<unsigned long long>(4, run.owned);
+        s.goss_rows = dalloc<int32_t>(ds->n, run.arena);
+        s.goss_max = dalloc<unsigned long long>(4, run.arena);
         HIPX(hipMemset(s.goss_max, 0, 4 * sizeof(unsigned long long)));
-        if (p->objective == MBH_OBJ_MULTICLASS) s.goss_imp = dalloc<double>(ds->n, run.owned);
+        if (p->objective == MBH_OBJ_MULTICLASS) s.goss_imp = dalloc<double>(ds->n, run.arena);
     }
     hp.bagging = (p->bagging_freq > 0 && p->bagging_fraction < 1.0) ? 1 : 0;
     hp.bagging_freq = p->bagging_freq;
@@ -714,7 +866,7 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
             }
             if (!any) fb[(size_t)b] = min_unit;
         }
-        int64_t *d_fb = dalloc<int64_t>(n_bags, run.owned);
+        int64_t *d_fb = dalloc<int64_t>(n_bags, run.arena);
         HIPX(hipMemcpy(d_fb, fb.data(), n_bags * sizeof(int64_t), hipMemcpyHostToDevice));
         s.bag_fallback = d_fb;
         s.n_bags = n_bags;
@@ -724,7 +876,7 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
             std::vector<int32_t> qid((size_t)ds->n);
             for (size_t q = 0; q + 1 < ds->qstart.size(); ++q)
                 for (int64_t r = ds->qstart[q]; r < ds->qstart[q + 1]; ++r) qid[(size_t)r] = (int32_t)q;
-            int32_t *d_qid = dalloc<int32_t>(ds->n, run.owned);
+            int32_t *d_qid = dalloc<int32_t>(ds->n, run.arena);
             HIPX(hipMemcpy(d_qid, qid.data(), (size_t)ds->n * sizeof(int32_t), hipMemcpyHostToDevice));
             s.qid = d_qid;
         }
@@ -741,7 +893,7 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
     hp.cat_l2 = p->cat_l2;
 
     // the fp32 path's binary32 derivatives, interleaved per row
-    if (!quantized && !hp.grad64) s.gh2 = dalloc<float>(2 * (size_t)ds->n, run.owned);
+    if (!quantized && !hp.grad64) s.gh2 = dalloc<float>(2 * (size_t)ds->n, run.arena);
     if (mb::plan_lds_bytes(s) > 160 * 1024)
         throw Error{MOJOTREES_ERROR_UNSUPPORTED,
                     "num_leaves * n_features too large for the planner's LDS (160 KiB)"};
@@ -800,9 +952,9 @@ void setup_record_partition(mb::DevState &s, const mbh_dataset *ds, const mbh_pa
     if (mode < 0 || mode > 2) throw Error{MOJOTREES_ERROR_INVALID_ARGUMENT, "partition_mode must be 0, 1 or 2"};
     s.rcp = eligible && mode == 1 ? 1 : 0;
     if (!s.rcp) return;
-    s.crec0 = dalloc<uint8_t>((size_t)ds->n * s.rec_bytes, run.owned);
-    s.crec1 = dalloc<uint8_t>((size_t)ds->n * s.rec_bytes, run.owned);
-    s.pairs = dalloc<uint16_t>(ds->n, run.owned);
+    s.crec0 = dalloc<uint8_t>((size_t)ds->n * s.rec_bytes, run.arena);
+    s.crec1 = dalloc<uint8_t>((size_t)ds->n * s.rec_bytes, run.arena);
+    s.pairs = dalloc<uint16_t>(ds->n, run.arena);
     // the root's batch shares the record partition's kPartChunk-row tasks
     // (16K-row tasks would hold 16 records per thread)
     s.part_root = 0;
@@ -824,64 +976,64 @@ mb::DevState clone_class_state(const mb::DevState &s0, const mbh_dataset *ds, in
     const int F = ds->F;
     s.hp.class_stride = stride;
     const size_t rec_total = (size_t)s0.n_tiles * (size_t)n * (size_t)s0.rec_bytes;
-    uint8_t *rec = dalloc<uint8_t>(rec_total, run.owned);
+    uint8_t *rec = dalloc<uint8_t>(rec_total, run.arena);
     HIPX(hipMemcpy(rec, s0.records, rec_total, hipMemcpyDeviceToDevice));
     s.records = rec;
     s.records_w = rec;
-    s.grad = dalloc<float>(n, run.owned);
-    s.hess = dalloc<float>(n, run.owned);
-    if (s0.gh2) s.gh2 = dalloc<float>(2 * (size_t)n, run.owned);
-    s.stats = dalloc<uint32_t>(4 * mb::kStatSlots, run.owned);
-    s.round = dalloc<mb::Round>(1, run.owned);
-    s.rows0 = dalloc<int32_t>(n, run.owned);
-    s.rows1 = dalloc<int32_t>(n, run.owned);
-    if (s0.hist) s.hist = dalloc<int32_t>((size_t)(1 + s0.max_exp) * F * ds->nb * 3, run.owned);
-    if (s0.histf) s.histf = dalloc<mb::HistF>((size_t)(1 + s0.max_exp) * F * ds->nb, run.owned);
+    s.grad = dalloc<float>(n, run.arena);
+    s.hess = dalloc<float>(n, run.arena);
+    if (s0.gh2) s.gh2 = dalloc<float>(2 * (size_t)n, run.arena);
+    s.stats = dalloc<uint32_t>(4 * mb::kStatSlots, run.arena);
+    s.round = dalloc<mb::Round>(1, run.arena);
+    s.rows0 = dalloc<int32_t>(n, run.arena);
+    s.rows1 = dalloc<int32_t>(n, run.arena);
+    if (s0.hist) s.hist = dalloc<int32_t>((size_t)(1 + s0.max_exp) * F * ds->nb * 3, run.arena);
+    if (s0.histf) s.histf = dalloc<mb::HistF>((size_t)(1 + s0.max_exp) * F * ds->nb, run.arena);
     const int kind = s0.hp.wide ? mb::kAccWide : s0.hp.quantized ? mb::kAccQuant : mb::kAccFloat;
     s.part = nullptr;
     s.part_c = nullptr;
     s.fpart_g = s.fpart_h = nullptr;
     s.fpart_c = nullptr;
     configure_hist(s, ds, s0.hp.quantized ? s0.hp.quant_bins : 4, kind, run);
-    if (s0.gq) s.gq = dalloc<int32_t>(2 * (size_t)n, run.owned);
-    if (s0.magpart) s.magpart = dalloc<float>(2 * 256, run.owned);
+    if (s0.gq) s.gq = dalloc<int32_t>(2 * (size_t)n, run.arena);
+    if (s0.magpart) s.magpart = dalloc<float>(2 * 256, run.arena);
     if (s0.stage16_over) {
-        s.stage16_over = dalloc<unsigned long long>(2, run.owned);
+        s.stage16_over = dalloc<unsigned long long>(2, run.arena);
         HIPX(hipMemset(s.stage16_over, 0, 2 * sizeof(unsigned long long)));
     }
     if (s0.goss_max) {
-        s.goss_max = dalloc<unsigned long long>(4, run.owned);
+        s.goss_max = dalloc<unsigned long long>(4, run.arena);
         HIPX(hipMemset(s.goss_max, 0, 4 * sizeof(unsigned long long)));
     }
-    s.enodes = dalloc<mb::ENode>(s.e_cap, run.owned);
-    s.items = dalloc<mb::Item>(s.kmax, run.owned);
-    s.batch = dalloc<mb::Batch>(1, run.owned);
-    s.grow = dalloc<mb::Grow>(1, run.owned);
-    s.slot_e = dalloc<int32_t>(L, run.owned);
-    s.slot_fid = dalloc<int32_t>(L, run.owned);
-    s.scan = dalloc<mb::ScanResult>((size_t)s.kmax * 2 * F, run.owned);
-    s.scan_gain = dalloc<double>((size_t)s.kmax * 2 * F, run.owned);
-    s.pair_gain = dalloc<double>((size_t)s.kmax * 2, run.owned);
-    s.pair_feat = dalloc<int32_t>((size_t)s.kmax * 2, run.owned);
-    s.e_gain = dalloc<double>(s.e_cap, run.owned);
-    s.e_left = dalloc<int32_t>(s.e_cap, run.owned);
-    s.e_rows = dalloc<int32_t>(s.e_cap, run.owned);
-    s.e_parent = dalloc<int32_t>(s.e_cap, run.owned);
-    s.cursor = dalloc<int64_t>(2 + 2 * (size_t)s.kmax, run.owned);
-    s.t_feature = dalloc<int32_t>(max_nodes, run.owned);
-    s.t_threshold = dalloc<int32_t>(max_nodes, run.owned);
-    s.t_left = dalloc<int32_t>(max_nodes, run.owned);
-    s.t_right = dalloc<int32_t>(max_nodes, run.owned);
-    s.t_default_left = dalloc<int32_t>(max_nodes, run.owned);
-    s.t_missing_bin = dalloc<int32_t>(max_nodes, run.owned);
-    s.t_value = dalloc<double>(max_nodes, run.owned);
-    s.t_gain = dalloc<double>(max_nodes, run.owned);
-    s.t_count = dalloc<double>(max_nodes, run.owned);
-    s.t_meta = dalloc<int32_t>(2, run.owned);
+    s.enodes = dalloc<mb::ENode>(s.e_cap, run.arena);
+    s.items = dalloc<mb::Item>(s.kmax, run.arena);
+    s.batch = dalloc<mb::Batch>(1, run.arena);
+    s.grow = dalloc<mb::Grow>(1, run.arena);
+    s.slot_e = dalloc<int32_t>(L, run.arena);
+    s.slot_fid = dalloc<int32_t>(L, run.arena);
+    s.scan = dalloc<mb::ScanResult>((size_t)s.kmax * 2 * F, run.arena);
+    s.scan_gain = dalloc<double>((size_t)s.kmax * 2 * F, run.arena);
+    s.pair_gain = dalloc<double>((size_t)s.kmax * 2, run.arena);
+    s.pair_feat = dalloc<int32_t>((size_t)s.kmax * 2, run.arena);
+    s.e_gain = dalloc<double>(s.e_cap, run.arena);
+    s.e_left = dalloc<int32_t>(s.e_cap, run.arena);
+    s.e_rows = dalloc<int32_t>(s.e_cap, run.arena);
+    s.e_parent = dalloc<int32_t>(s.e_cap, run.arena);
+    s.cursor = dalloc<int64_t>(2 + 2 * (size_t)s.kmax, run.arena);
+    s.t_feature = dalloc<int32_t>(max_nodes, run.arena);
+    s.t_threshold = dalloc<int32_t>(max_nodes, run.arena);
+    s.t_left = dalloc<int32_t>(max_nodes, run.arena);
+    s.t_right = dalloc<int32_t>(max_nodes, run.arena);
+    s.t_default_left = dalloc<int32_t>(max_nodes, run.arena);
+    s.t_missing_bin = dalloc<int32_t>(max_nodes, run.arena);
+    s.t_value = dalloc<double>(max_nodes, run.arena);
+    s.t_gain = dalloc<double>(max_nodes, run.arena);
+    s.t_count = dalloc<double>(max_nodes, run.arena);
+    s.t_meta = dalloc<int32_t>(2, run.arena);
     if (s0.scan_cat) {
-        s.scan_cat = dalloc<unsigned long long>((size_t)s.kmax * 2 * F * 4, run.owned);
-        s.e_cat = dalloc<unsigned long long>((size_t)s.e_cap * 4, run.owned);
-        s.t_cat = dalloc<unsigned long long>((size_t)max_nodes * 4, run.owned);
+        s.scan_cat = dalloc<unsigned long long>((size_t)s.kmax * 2 * F * 4, run.arena);
+        s.e_cat = dalloc<unsigned long long>((size_t)s.e_cap * 4, run.arena);
+        s.t_cat = dalloc<unsigned long long>((size_t)max_nodes * 4, run.arena);
         HIPX(hipMemset(s.t_cat, 0, (size_t)max_nodes * 4 * sizeof(unsigned long long)));
     }
     HIPX(hipMemset(s.rows0, 0, (size_t)n * sizeof(int32_t)));
@@ -1097,7 +1249,7 @@ int32_t mbh_train(mbh_dataset *ds, const mbh_params *p, mbh_fit **out, char *err
     std::vector<hipEvent_t> events;
     try {
         check_params(ds, p);
-        Run run;
+        Run run(ds);
         TrainBuffers tb = setup_state(ds, p, run);
         mb::DevState &s = tb.s;
         setup_record_partition(s, ds, p, run);
@@ -1107,7 +1259,7 @@ int32_t mbh_train(mbh_dataset *ds, const mbh_params *p, mbh_fit **out, char *err
         fit->n_features = ds->F;
         fit->learning_rate = p->learning_rate;
         fit->base = base_scores_for(ds, p->objective, K);
-        double *d_base = dalloc<double>(K, run.owned);
+        double *d_base = dalloc<double>(K, run.arena);
         HIPX(hipMemcpy(d_base, fit->base.data(), K * sizeof(double), hipMemcpyHostToDevice));
         const int grid_rows = 8 * ds->n_cu;
         HIPX(mb::launch_fill_f64(s.raw, ds->n, K, d_base, grid_rows, nullptr));
@@ -1158,7 +1310,7 @@ int32_t mbh_train(mbh_dataset *ds, const mbh_params *p, mbh_fit **out, char *err
         };
         if (timed) {
             s.iter_stride = L + kMaxGroup + 4;
-            s.iter_log = dalloc<int64_t>((size_t)T * s.iter_stride * 2, run.owned);
+            s.iter_log = dalloc<int64_t>((size_t)T * s.iter_stride * 2, run.arena);
             HIPX(hipMemset(s.iter_log, 0, (size_t)T * s.iter_stride * 2 * sizeof(int64_t)));
         }
         // expansion launches the previous tree needed: the first group of a
@@ -1404,14 +1556,15 @@ int32_t mbh_train(mbh_dataset *ds, const mbh_params *p, mbh_fit **out, char *err
             acat.resize((size_t)tb.T * mn * 4);
             HIPX(hipMemcpy(acat.data(), s.arc_cat, acat.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost));
         }
-        fit->train_raw.resize((size_t)ds->n * K);
-        HIPX(hipMemcpy(fit->train_raw.data(), s.raw, fit->train_raw.size() * sizeof(double),
-                       hipMemcpyDeviceToHost));
-        if (K > 1) {  // the device's class-major scores to the row-major layout of the API
-            std::vector<double> cm(fit->train_raw);
-            for (int64_t r = 0; r < ds->n; ++r)
-                for (int k = 0; k < K; ++k) fit->train_raw[(size_t)r * K + k] = cm[(size_t)k * ds->n + r];
+        // the device's class-major scores in the row-major layout of the API
+        // (into the probabilities' buffer, free now)
+        const double *scores = s.raw;
+        if (K > 1) {
+            HIPX(mb::launch_row_major(s.raw, s.prob, ds->n, K, nullptr));
+            scores = s.prob;
         }
+        fit->train_raw.reserve((size_t)ds->n * K);
+        HIPX(hipMemcpy(fit->train_raw.p, scores, fit->train_raw.n * sizeof(double), hipMemcpyDeviceToHost));
         const bool bagging = s.hp.bagging != 0 || s.hp.goss != 0;  // sampled rounds are skipped, not stops
         // algorithmic bytes per accumulated row: its bins plus its g/h pair
         // (int8 x 2 quantized, fp32 x 2 otherwise)
@@ -1516,6 +1669,11 @@ int32_t mbh_train(mbh_dataset *ds, const mbh_params *p, mbh_fit **out, char *err
         set_err(err, err_len, e.msg);
         delete fit;
         return e.code;
+    } catch (const std::exception &e) {  // host memory
+        for (auto &ev : events) (void)hipEventDestroy(ev);
+        set_err(err, err_len, e.what());
+        delete fit;
+        return MOJOTREES_ERROR_TRAINING;
     }
     *out = fit;
     return MOJOTREES_OK;
@@ -1549,7 +1707,7 @@ int32_t mbh_fit_train_raw(const mbh_fit *fit, double *out, char *err, int32_t er
         set_err(err, err_len, "null argument");
         return MOJOTREES_ERROR_INVALID_ARGUMENT;
     }
-    std::memcpy(out, fit->train_raw.data(), fit->train_raw.size() * sizeof(double));
+    std::memcpy(out, fit->train_raw.p, fit->train_raw.n * sizeof(double));
     return MOJOTREES_OK;
 }
 int64_t mbh_fit_launch_log(const mbh_fit *fit, double *out, int64_t n_out) {
@@ -1575,10 +1733,10 @@ int32_t mbh_exp_sigmoid(const double *x, int64_t n, double *out_exp, double *out
         set_err(err, err_len, "no gfx950 device");
         return MOJOTREES_ERROR_UNSUPPORTED;
     }
-    Run run;
+    Run run(nullptr);
     try {
-        double *dx = dalloc<double>(n, run.owned), *de = dalloc<double>(n, run.owned),
-               *dsg = dalloc<double>(n, run.owned);
+        double *dx = dalloc<double>(n, run.arena), *de = dalloc<double>(n, run.arena),
+               *dsg = dalloc<double>(n, run.arena);
         HIPX(hipMemcpy(dx, x, n * sizeof(double), hipMemcpyHostToDevice));
         HIPX(mb::launch_exp_sigmoid(dx, de, dsg, n, nullptr));
         HIPX(hipMemcpy(out_exp, de, n * sizeof(double), hipMemcpyDeviceToHost));
@@ -1676,7 +1834,7 @@ int32_t mbh_lambdarank(mbh_dataset *ds, const mbh_params *p, const double *raw, 
         p1.objective = MBH_OBJ_LAMBDARANK;
         p1.num_iterations = 1;
         check_params(ds, &p1);
-        Run run;
+        Run run(ds);
         TrainBuffers tb = setup_state(ds, &p1, run);
         mb::DevState &s = tb.s;
         HIPX(hipMemcpy(s.raw, raw, ds->n * sizeof(double), hipMemcpyHostToDevice));
@@ -1701,7 +1859,7 @@ int32_t mbh_objective_quantize(mbh_dataset *ds, const mbh_params *p, const doubl
     }
     try {
         check_params(ds, p);
-        Run run;
+        Run run(ds);
         mbh_params p1 = *p;
         p1.num_iterations = 1;
         if (round_index < 0) throw Error{MOJOTREES_ERROR_INVALID_ARGUMENT, "round_index must be nonnegative"};
@@ -1744,7 +1902,7 @@ int32_t mbh_objective_quantize32(mbh_dataset *ds, const mbh_params *p, const dou
     try {
         if (!p->use_quantized_grad) throw Error{MOJOTREES_ERROR_INVALID_ARGUMENT, "use_quantized_grad must be 1"};
         check_params(ds, p);
-        Run run;
+        Run run(ds);
         mbh_params p1 = *p;
         p1.num_iterations = 1;
         if (round_index < 0) throw Error{MOJOTREES_ERROR_INVALID_ARGUMENT, "round_index must be nonnegative"};
@@ -1838,7 +1996,7 @@ int32_t mbh_histogram32(mbh_dataset *ds, const int32_t *q_grad, const int32_t *q
         }
         if (sg >= ((int64_t)1 << 31) || sh >= ((int64_t)1 << 31))
             throw Error{MOJOTREES_ERROR_INVALID_ARGUMENT, "the selection's quantized magnitudes exceed int32 cells"};
-        Run run;
+        Run run(ds);
         mbh_params p{};
         p.objective = MBH_OBJ_BINARY;
         p.num_iterations = 1;
@@ -1895,7 +2053,7 @@ int32_t mbh_histogram(mbh_dataset *ds, const int8_t *q_grad, const int8_t *q_hes
         for (int64_t r = 0; r < ds->n; ++r)
             if (q_grad[r] < -(B / 2 + 1) || q_grad[r] > B / 2 + 1 || q_hess[r] < 0 || q_hess[r] > B + 1)
                 throw Error{MOJOTREES_ERROR_INVALID_ARGUMENT, "quantized value outside the lattice"};
-        Run run;
+        Run run(ds);
         mbh_params p{};
         p.objective = MBH_OBJ_BINARY;
         p.num_iterations = 1;
@@ -1953,7 +2111,7 @@ int32_t mbh_histogram_fp32(mbh_dataset *ds, const float *grad, const float *hess
             for (int64_t i = 0; i < n_sel; ++i)
                 if (rows[i] < 0 || rows[i] >= ds->n)
                     throw Error{MOJOTREES_ERROR_INVALID_ARGUMENT, "row id out of range"};
-        Run run;
+        Run run(ds);
         mbh_params p{};
         p.objective = MBH_OBJ_REGRESSION;
         p.num_iterations = 1;
@@ -2004,7 +2162,7 @@ int32_t mbh_bench_root_histogram(mbh_dataset *ds, int32_t reps, double *out_ms, 
     }
     std::vector<hipEvent_t> ev((size_t)3 * reps);
     try {
-        Run run;
+        Run run(ds);
         mbh_params p{};
         p.objective = MBH_OBJ_BINARY;
         p.num_iterations = 1;

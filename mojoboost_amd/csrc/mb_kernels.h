@@ -56,6 +56,8 @@ enum RowsKernel { kRowsScore = 0, kRowsScoreObjective = 1, kRowsSoftmax = 2 };
 int rows_grid(const DevState &s, RowsKernel k, int n_cu);
 hipError_t launch_build_records(const uint8_t *bins_cm, uint8_t *records, int64_t n, int F, int rec,
                                 int tile_f, int n_tiles, int grid, hipStream_t st);
+// n x K row-major from class-major scores.
+hipError_t launch_row_major(const double *in, double *out, int64_t n, int K, hipStream_t st);
 hipError_t launch_fill_f64(double *p, int64_t n, int K, const double *base, int grid, hipStream_t st);
 hipError_t launch_exp_sigmoid(const double *x, double *e, double *sg, int64_t n, hipStream_t st);
 

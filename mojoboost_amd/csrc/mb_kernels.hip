@@ -5761,6 +5761,25 @@ __global__ __launch_bounds__(256) void k_build_records(const uint8_t *bins_cm, u
     }
 }
 
+// Class-major scores (class k of row r at k n + r) to row-major ones: 64 rows
+// of a block through LDS, a run of classes at a time, so both sides move
+// consecutive values.
+constexpr int kRowMajorK = 16;
+__global__ __launch_bounds__(256) void k_row_major(const double *__restrict__ in, double *__restrict__ out, int64_t n,
+                                                   int K) {
+    __shared__ double t[64][kRowMajorK + 1];
+    const int64_t r0 = (int64_t)blockIdx.x * 64;
+    const int rows = (int)(n - r0 < 64 ? n - r0 : 64);
+    const int k0 = (int)blockIdx.y * kRowMajorK, ks = min(kRowMajorK, K - k0);
+    for (int i = threadIdx.x; i < 64 * ks; i += 256)
+        if ((i & 63) < rows) t[i & 63][i >> 6] = in[(size_t)(k0 + (i >> 6)) * n + r0 + (i & 63)];
+    __syncthreads();
+    for (int i = threadIdx.x; i < rows * ks; i += 256) {
+        const int r = i / ks, k = i - r * ks;
+        out[(size_t)(r0 + r) * K + k0 + k] = t[r][k];
+    }
+}
+
 // The initial raw scores, class-major: class k of row r at k n + r.
 __global__ __launch_bounds__(256) void k_fill_f64(double *p, int64_t n, int K, const double *base) {
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -6056,6 +6075,11 @@ hipError_t launch_build_records(const uint8_t *bins_cm, uint8_t *records, int64_
                                 int tile_f, int n_tiles, int grid, hipStream_t st) {
     hipLaunchKernelGGL(k_build_records, dim3(grid), dim3(256), 0, st, bins_cm, records, n, F, rec, tile_f,
                        n_tiles);
+    return hipGetLastError();
+}
+hipError_t launch_row_major(const double *in, double *out, int64_t n, int K, hipStream_t st) {
+    hipLaunchKernelGGL(k_row_major, dim3((unsigned)((n + 63) / 64), (unsigned)((K + kRowMajorK - 1) / kRowMajorK)),
+                       dim3(256), 0, st, in, out, n, K);
     return hipGetLastError();
 }
 hipError_t launch_fill_f64(double *p, int64_t n, int K, const double *base, int grid, hipStream_t st) {
