@@ -1931,7 +1931,8 @@ struct QAcc {
         return (size_t)row_cells_for(record_bytes_for(tf)) * ls * 8;
     }
     template <int LPR>
-    __device__ static void zero(unsigned char *lds, int, int ls) {
+    __device__ static void zero(unsigned char *lds, const DevState &s) {
+        const int ls = s.lds_stride;
         constexpr int FS = row_cells_for(LPR * 16);
         unsigned long long *a = (unsigned long long *)lds;
         for (int i = threadIdx.x; i < FS * ls; i += blockDim.x) a[i] = 0ULL;
@@ -1944,8 +1945,7 @@ struct QAcc {
     // over 32 banks), and the 32 lanes of a half-wave 32 different positions
     // mod 32 (none when it serves 32 lanes over 64 banks), for LPR >= 2.
     template <int LPR>
-    __device__ static void add(unsigned char *lds, const DevState &, const uint4 &w, int sub, int, int, int64_t,
-                               uint32_t gh_word, double) {
+    __device__ static void add(unsigned char *lds, const uint4 &w, int sub, uint32_t gh_word) {
         constexpr int FS = row_cells_for(LPR * 16);
         constexpr int kRowShift = FS == 32 ? 8 : FS == 64 ? 9 : 10;  // log2(FS * 8 bytes)
         static_assert(FS * 8 == (1 << kRowShift), "row of a power-of-two size");
@@ -2012,7 +2012,8 @@ struct FAcc {
         return (size_t)2 * FS * ls * 8 + (size_t)count_rows(ls) * FS * 4;
     }
     template <int LPR>
-    __device__ static void zero(unsigned char *lds, int, int ls) {
+    __device__ static void zero(unsigned char *lds, const DevState &s) {
+        const int ls = s.lds_stride;
         constexpr int FS = QAcc::row_cells_for(LPR * 16);
         double *g = (double *)lds;
         uint32_t *c = (uint32_t *)(g + 2 * (size_t)FS * ls);
@@ -2083,60 +2084,89 @@ struct FAcc {
 };
 
 // WAcc (the magnitude-sum lattice): each row's int32 (grad, hess) pair from
-// `gq`, gathered by row id -- or, with int16 staging (K16), the int16 pair in
-// the record's last four bytes, which the row's lanes already hold; per cell
-// one 64-bit LDS add of the packed pair --
+// `gq`, gathered by row id with the record a step ahead -- or, with int16
+// staging (K16), the int16 pair in the record's last four bytes, which the
+// row's lanes already hold; per cell one 64-bit LDS add of the packed pair --
 // hess in the low 32 bits (nonnegative, a cell's sum below 2^32), signed grad
 // in the high 32 -- and one 32-bit count. Any subset of a round's rows sums
 // to at most 2^30 + n in magnitude on this lattice (quantized_gradient.mojo:
 // 908-1117, the headroom argument), so neither field overflows and no carry
 // crosses from hess into grad, whatever the block's row count.
+// Cells are bin-major over FS byte positions, as QAcc's, where that fits a
+// workgroup's LDS (at 255 bins, tiles of at most 28 features), else
+// feature-major (up to 52 of them, the lanes of a step on random banks).
+struct WCells {
+    int sb, sp, total;  // cell (bin, position) at bin * sb + position * sp
+};
+__host__ __device__ inline WCells wide_cells(int tf, int ls) {
+    const int FS = QAcc::row_cells_for(record_bytes_for(tf + 2));
+    if ((size_t)FS * ls * 12 <= 156 * 1024) return WCells{FS, 1, FS * ls};
+    return WCells{1, ls, tf * ls};
+}
 template <bool K16>
 struct WAccT {
-    static __host__ __device__ size_t lds_bytes(int F, int ls) { return (size_t)F * ls * 12; }
+    static __host__ __device__ size_t lds_bytes(int tf, int ls) { return (size_t)wide_cells(tf, ls).total * 12; }
     template <int LPR>
-    __device__ static void zero(unsigned char *lds, int F, int ls) {
+    __device__ static void zero(unsigned char *lds, const DevState &s) {
+        const int n = wide_cells(s.tile_f, s.lds_stride).total;
         unsigned long long *gh = (unsigned long long *)lds;
-        uint32_t *c = (uint32_t *)(gh + (size_t)F * ls);
-        for (int i = threadIdx.x; i < F * ls; i += blockDim.x) {
+        uint32_t *c = (uint32_t *)(gh + n);
+        for (int i = threadIdx.x; i < n; i += blockDim.x) {
             gh[i] = 0ULL;
             c[i] = 0u;
         }
     }
+    // pair: the row's int32 pair, grad in the high half
     template <int LPR>
-    __device__ static void add(unsigned char *lds, const DevState &s, const uint4 &w, int sub, int F, int ls,
-                               int64_t row, uint32_t gh_word, double) {
+    __device__ static void add(unsigned char *lds, const DevState &s, const uint4 &w, int sub, int F,
+                               unsigned long long pair, uint32_t gh_word) {
+        const WCells wc = wide_cells(s.tile_f, s.lds_stride);
         unsigned long long *gh = (unsigned long long *)lds;
-        uint32_t *c = (uint32_t *)(gh + (size_t)F * ls);
-        int2 q;
-        if constexpr (K16) q = make_int2((int)(int16_t)(gh_word & 0xFFFFu), (int)(int16_t)(gh_word >> 16));
-        else q = *(const int2 *)(s.gq + 2 * row);
-        const unsigned long long packed = ((unsigned long long)(uint32_t)q.x << 32) | (uint32_t)q.y;
-        const uint32_t d[4] = {w.x, w.y, w.z, w.w};
+        uint32_t *c = (uint32_t *)(gh + wc.total);
+        if constexpr (K16)
+            pair = ((unsigned long long)(uint32_t)(int32_t)(int16_t)(gh_word & 0xFFFFu) << 32) |
+                   (uint32_t)(int32_t)(int16_t)(gh_word >> 16);
+        const uint32_t rot = ((uint32_t)lane_id() & 15u) ^ (((uint32_t)lane_id() >> 4) & 1u);
+        uint32_t r[4];
+        rotate_slice(w.x, w.y, w.z, w.w, rot, r);
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int f = sub * 16 + k * 4 + j;
-                if (f < F) {
-                    const int cell = f * ls + (int)((d[k] >> (8 * j)) & 255u);
-                    atomicAdd(&gh[cell], packed);
-                    atomicAdd(&c[cell], 1u);
-                }
+        for (int k = 0; k < 16; ++k) {
+            const int p = sub * 16 + (int)(((uint32_t)k + rot) & 15u);
+            const int bin = (int)((r[k >> 2] >> (8 * (k & 3))) & 255u);
+            if (p < F) {
+                const int cell = bin * wc.sb + p * wc.sp;
+                atomicAdd(&gh[cell], pair);
+                atomicAdd(&c[cell], 1u);
             }
+        }
     }
+    // feature-major partials; a lane takes four bins of one feature, as
+    // QAcc::store
     template <int LPR>
     __device__ static void store(const DevState &s, const unsigned char *lds, int blk, int f0, int Ft) {
-        const int F = s.n_features, nb = s.n_bins, ls = s.lds_stride, ps = s.part_stride;
+        const WCells wc = wide_cells(s.tile_f, s.lds_stride);
+        const int F = s.n_features, nb = s.n_bins, ps = s.part_stride;
         const unsigned long long *gh = (const unsigned long long *)lds;
-        const uint32_t *c = (const uint32_t *)(gh + (size_t)Ft * ls);
+        const uint32_t *c = (const uint32_t *)(gh + wc.total);
         const size_t base = ((size_t)blk * F + f0) * ps;
-        for (int i = threadIdx.x; i < Ft * ps; i += blockDim.x) {
-            const int f = i / ps;
-            const int b = i - f * ps;
-            const bool in = b < nb;
-            s.part[base + i] = in ? gh[f * ls + b] : 0ULL;
-            s.part_c[base + i] = in ? c[f * ls + b] : 0u;
+        const int nq = (ps + 3) >> 2;
+        for (int u = threadIdx.x; u < Ft * nq; u += blockDim.x) {
+            const int q = u / Ft, f = u - q * Ft, b = 4 * q;
+            unsigned long long v[4];
+            uint32_t vc[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int cell = (b + i) * wc.sb + f * wc.sp;
+                v[i] = b + i < nb ? gh[cell] : 0ULL;
+                vc[i] = b + i < nb ? c[cell] : 0u;
+            }
+            const size_t o = base + (size_t)f * ps + b;  // ps is even: 16-byte aligned pairs
+            *(ulonglong2 *)(s.part + o) = make_ulonglong2(v[0], v[1]);
+            *(uint2 *)(s.part_c + o) = make_uint2(vc[0], vc[1]);
+            if (b + 2 < ps) {
+                *(ulonglong2 *)(s.part + o + 2) = make_ulonglong2(v[2], v[3]);
+                *(uint2 *)(s.part_c + o + 2) = make_uint2(vc[2], vc[3]);
+            }
         }
     }
 };
@@ -2241,6 +2271,10 @@ __device__ __forceinline__ void accumulate_rows(const DevState &s, unsigned char
     // binary32 derivatives come as one interleaved (g, h) pair whose h sign
     // bit carries the GOSS weight bit (one gather per row, not three)
     constexpr bool kF = std::is_same<Acc, FAcc>::value;
+    // the magnitude-sum lattice's cells: the row's int32 pair (in fg, grad in
+    // the high half), loaded with the record likewise
+    constexpr bool kG = std::is_same<Acc, WAcc>::value;
+    constexpr bool kW = kG || std::is_same<Acc, WAcc16>::value;
     const bool f64 = kF && s.hp.grad64;
     const bool f_goss = kF && goss_mult != 1.0 && (f64 ? s.goss_other != nullptr : true);
     unsigned long long fg[U], fh[U], fg_nxt[U], fh_nxt[U];
@@ -2257,6 +2291,10 @@ __device__ __forceinline__ void accumulate_rows(const DevState &s, unsigned char
                 v[u] = (LPR == 1 || (sub & 1) == 0) ? s.grad[r] : s.hess[r];
                 if constexpr (LPR == 1) v2[u] = s.hess[r];
                 if (q_goss) wb |= (s.goss_other[r] ? 1u : 0u) << u;
+            }
+            if constexpr (kG) {
+                const uint2 q = ((const uint2 *)s.gq)[r];
+                xg[u] = ((unsigned long long)q.x << 32) | q.y;
             }
             if constexpr (kF) {
                 if (f64) {
@@ -2335,8 +2373,10 @@ __device__ __forceinline__ void accumulate_rows(const DevState &s, unsigned char
                 }
                 if (i < hi) FAcc::template add<LPR>(lds, w[u], sub, Ft, ls, gv, hv);
             } else {
-                if (i < hi)
-                    Acc::template add<LPR>(lds, s, w[u], sub, Ft, ls, (int64_t)(uint32_t)id[u], gh[u], goss_mult);
+                if (i < hi) {
+                    if constexpr (kW) Acc::template add<LPR>(lds, s, w[u], sub, Ft, xg[u], gh[u]);
+                    else Acc::template add<LPR>(lds, w[u], sub, gh[u]);
+                }
             }
         }
     };
@@ -2367,10 +2407,8 @@ __device__ __forceinline__ void accumulate_rows(const DevState &s, unsigned char
                 qv[u] = qv_nxt[u];
                 if constexpr (LPR == 1) qv2[u] = qv2_nxt[u];
             }
-            if constexpr (kF) {
-                fg[u] = fg_nxt[u];
-                fh[u] = fh_nxt[u];
-            }
+            if constexpr (kF || kG) fg[u] = fg_nxt[u];
+            if constexpr (kF) fh[u] = fh_nxt[u];
         }
         qw = qw_nxt;
         fw = fw_nxt;
@@ -2392,7 +2430,7 @@ __global__ __launch_bounds__(1024) void k_hist(DevState s) {
     const int ls = s.lds_stride;
     const int f0 = (int)blockIdx.y * s.tile_f;
     const int Ft = min(s.tile_f, s.n_features - f0);
-    Acc::template zero<LPR>(lds, Ft, ls);
+    Acc::template zero<LPR>(lds, s);
     __syncthreads();
     const uint4 *rec = (const uint4 *)(s.records + (size_t)blockIdx.y * s.n * s.rec_bytes);
     if constexpr (kQ) {
@@ -2799,7 +2837,7 @@ __global__ __launch_bounds__(kAccThreads) void k_accum(DevState s) {
         // the histogram is zeroed while the task's first records load
         accumulate_rows<LPR, Acc, true, false, std::is_same<Acc, FAcc>::value ? kAccUnrollF : kAccUnroll>(
             s, lds, buf ? s.rows1 : s.rows0, lo, hi, Ft, rec, goss_mult, nullptr, nullptr, [&]() {
-                Acc::template zero<LPR>(lds, Ft, ls);
+                Acc::template zero<LPR>(lds, s);
                 __syncthreads();
             });
         __syncthreads();
@@ -2834,7 +2872,7 @@ __global__ __launch_bounds__(kAccThreads) void k_accum_rec(DevState s) {
         const int64_t hi = lo + bh.chunk_a < hi_item ? lo + bh.chunk_a : hi_item;
         const int buf = __builtin_amdgcn_readlane(ait.buf, q);
         const uint4 *rec = (const uint4 *)(buf ? s.crec1 : s.crec0);
-        QAcc::template zero<LPR>(lds, Ft, ls);
+        QAcc::template zero<LPR>(lds, s);
         __syncthreads();
         accumulate_rows<LPR, QAcc, false, false, kAccUnrollRec>(s, lds, nullptr, lo, hi, Ft, rec, 1.0);
         __syncthreads();
@@ -2867,7 +2905,8 @@ __device__ __forceinline__ double readlane_f64_early(double d, int l) {
 // kCat: the dataset has categorical features (the category-set search is
 // compiled in). At most 128 VGPRs (4 waves per SIMD): two 512-thread blocks
 // per CU, so a batch's (leaf, feature) tasks need half the block rounds.
-template <bool kCat>
+// kWide: the magnitude-sum lattice's partials (a count plane beside the sums).
+template <bool kCat, bool kWide>
 __global__ __launch_bounds__(kScanThreads, 4) void k_scan(DevState s, int root_mode) {
     __shared__ int cg[2][256], ch[2][256], cc[2][256];
     __shared__ int acc[3][256];
@@ -2952,13 +2991,29 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan(DevState s, int root_m
                     s.part + (size_t)it.part_off * pstride + (size_t)f * s.part_stride + bin;
                 const int np = it.part_cnt;
                 int b = half;
-                if (hp.wide) {
+                if constexpr (kWide) {
                     // grad | hess halves and a separate count per partial
                     // (WAcc); the sums wrap as unsigned words, and every
                     // subset of the round's rows fits int32
                     const uint32_t *pc =
                         s.part_c + (size_t)it.part_off * pstride + (size_t)f * s.part_stride + bin;
                     uint32_t ug = 0u, uh = 0u, uc = 0u;
+                    // four partials' loads in flight (eight spill)
+                    for (; b + 6 < np; b += 8) {
+                        unsigned long long vv[4];
+                        uint32_t cv[4];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            vv[u] = p[(size_t)(b + 2 * u) * pstride];
+                            cv[u] = pc[(size_t)(b + 2 * u) * pstride];
+                        }
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            ug += (uint32_t)(vv[u] >> 32);
+                            uh += (uint32_t)vv[u];
+                            uc += cv[u];
+                        }
+                    }
                     for (; b < np; b += 2) {
                         const unsigned long long vv = p[(size_t)b * pstride];
                         ug += (uint32_t)(vv >> 32);
@@ -3377,6 +3432,7 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan(DevState s, int root_m
 // child's prefix sums are one wave scan and its best split one wave argmax,
 // with no block barrier. Candidates, guards and tie rules are k_scan's.
 constexpr int kNarrowFeat = kScanThreads / 128;
+template <bool kWide>
 __global__ __launch_bounds__(kScanThreads, 4) void k_scan_narrow(DevState s, int root_mode) {
     __shared__ int acc[kNarrowFeat][3][64];
     __shared__ int cv[kNarrowFeat][2][3][64];  // (g, h, c) of the accumulated child (0) and the sibling (1)
@@ -3462,10 +3518,26 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan_narrow(DevState s, int
                     s.part + (size_t)it.part_off * pstride + (size_t)f * s.part_stride + bin;
                 const int np = it.part_cnt;
                 int b = half;
-                if (hp.wide) {
+                if constexpr (kWide) {
                     const uint32_t *pc =
                         s.part_c + (size_t)it.part_off * pstride + (size_t)f * s.part_stride + bin;
                     uint32_t ug = 0u, uh = 0u, uc = 0u;
+                    // four partials' loads in flight (eight spill)
+                    for (; b + 6 < np; b += 8) {
+                        unsigned long long vv[4];
+                        uint32_t cv[4];
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            vv[u] = p[(size_t)(b + 2 * u) * pstride];
+                            cv[u] = pc[(size_t)(b + 2 * u) * pstride];
+                        }
+#pragma unroll
+                        for (int u = 0; u < 4; ++u) {
+                            ug += (uint32_t)(vv[u] >> 32);
+                            uh += (uint32_t)vv[u];
+                            uc += cv[u];
+                        }
+                    }
                     for (; b < np; b += 2) {
                         const unsigned long long vv = p[(size_t)b * pstride];
                         ug += (uint32_t)(vv >> 32);
@@ -6019,14 +6091,17 @@ hipError_t launch_scan(const DevState &s, int root_mode, hipStream_t st) {
     if (s.hp.quantized && !s.ncat && s.n_bins <= 64) {
         const int groups = (s.n_features + kNarrowFeat - 1) / kNarrowFeat;
         const int grid = root_mode ? groups : std::min(s.scan_grid, s.kmax * groups);
-        hipLaunchKernelGGL(k_scan_narrow, dim3(grid), dim3(kScanThreads), 0, st, s, root_mode);
+        hipLaunchKernelGGL(s.hp.wide ? k_scan_narrow<true> : k_scan_narrow<false>, dim3(grid), dim3(kScanThreads), 0, st,
+                           s, root_mode);
         return launch_fold(s, root_mode, st);
     }
     const int grid = root_mode ? s.n_features : s.scan_grid;
     if (s.hp.quantized && s.ncat)
-        hipLaunchKernelGGL(k_scan<true>, dim3(grid), dim3(kScanThreads), 0, st, s, root_mode);
+        hipLaunchKernelGGL((s.hp.wide ? k_scan<true, true> : k_scan<true, false>), dim3(grid), dim3(kScanThreads), 0, st,
+                           s, root_mode);
     else if (s.hp.quantized)
-        hipLaunchKernelGGL(k_scan<false>, dim3(grid), dim3(kScanThreads), 0, st, s, root_mode);
+        hipLaunchKernelGGL((s.hp.wide ? k_scan<false, true> : k_scan<false, false>), dim3(grid), dim3(kScanThreads), 0, st,
+                           s, root_mode);
     else if (s.ncat)
         hipLaunchKernelGGL(k_scan_f<true>, dim3(grid), dim3(kScanThreads), 0, st, s, root_mode);
     else
