@@ -549,6 +549,14 @@ void configure_hist(mb::DevState &s, const mbh_dataset *ds, int B, int kind, Run
     // the feature tiles)
     s.pb_launch = (int32_t)std::min<int64_t>((kind == mb::kAccFloat ? 1 : 2) * ds->n_cu,
                                              (ds->n + s.hist_chunk_min - 1) / s.hist_chunk_min + s.kmax);
+    // batches of few tasks are split into feature slices while that many
+    // blocks fit the chip at once (not the int8 lattice's: its histogram costs
+    // a task 2 us, and the sliced path's registers its second block per CU)
+    const int64_t tasks = (ds->n + s.hist_chunk_min - 1) / s.hist_chunk_min;
+    s.acc_slices = kind == mb::kAccQuant ? 1 : (s.tile_f + mb::kSliceF - 1) / mb::kSliceF;
+    s.slice_blocks = ds->n_cu;
+    s.acc_launch = std::max(s.pb_launch, (int32_t)std::min<int64_t>(ds->n_cu, (tasks + s.kmax) * s.acc_slices));
+    s.hist_slices = std::min(grid, tasks) * s.acc_slices * s.n_tiles <= 2 * ds->n_cu ? s.acc_slices : 1;
     // a batch's accumulation tasks: with chunk >= its rows / pb_launch (or
     // = limit) an item of m rows takes at most m / chunk + 1 of them
     s.pb_grid = (int32_t)(s.pb_launch + s.kmax + (ds->n + limit - 1) / limit);

@@ -85,7 +85,7 @@ struct Batch {
     int32_t n_acc;     // accumulation tasks (block partials) in use
     int32_t chunk_p;   // parent rows per partition task
     int32_t chunk_a;   // accumulated rows per accumulation task
-    int32_t pad_;
+    int32_t slices;    // feature slices an accumulation task is split into (1: none)
 };
 
 // Replay state of the best-first order (touched by the planning block only).
@@ -142,6 +142,8 @@ constexpr int kPartChunk = MB_PART_CHUNK;
 #endif
 constexpr int kPartChunkMin = MB_PART_CHUNK_MIN;
 constexpr int kPartChunkStep = 256;
+// Features of a slice of an accumulation task (small batches, k_accum).
+constexpr int kSliceF = 8;
 // Rows one fp32-path histogram block may add: its counts are 16-bit halves
 // of 32-bit LDS cells.
 constexpr int64_t kFAccChunk = 65535;
@@ -394,6 +396,10 @@ struct DevState {
     int32_t part_grid;     // most partition tasks of a batch
     int32_t scan_grid;     // blocks of a scan launch
     int32_t pb_launch;     // blocks of an accumulation launch (grid-strided)
+    int32_t acc_launch;    // blocks (x) of an accumulation launch: pb_launch, or more for slices
+    int32_t acc_slices;    // slices of a feature tile (1: never sliced)
+    int32_t slice_blocks;  // a batch is sliced when its tasks x slices x tiles are at most these
+    int32_t hist_slices;   // slices of the root build (1: none)
     int32_t part_launch;   // blocks of a partition launch (grid-strided)
     int32_t part_target;   // partition tasks a batch is spread over
     int32_t part_root;     // 1: the root's batch takes its own launch of kPartChunkRoot-row tasks
