@@ -519,7 +519,14 @@ void ensure_records(mbh_dataset *ds, const RecLayout &l) {
 constexpr int64_t kHistChunkMin = 2048;
 constexpr int64_t kHistChunkMinF = 1536;  // fp32 cells
 
-void configure_hist(mb::DevState &s, const mbh_dataset *ds, int B, int kind, Run &run) {
+// Rows and feature slices up to which one launch per iteration partitions and
+// accumulates (k_expand, which has both sides' figures).
+constexpr int64_t kExpandRows = 65536;
+constexpr int kExpandSlices = 6;
+
+// allow_expand: the run may use k_expand (not with per-kernel timing or
+// records in the leaves).
+void configure_hist(mb::DevState &s, const mbh_dataset *ds, int B, int kind, bool allow_expand, Run &run) {
     const bool quantized = kind != mb::kAccFloat;
     // the packed int8-lattice counters bound a block's rows; the other
     // accumulators hold whole-round sums in every field
@@ -564,6 +571,15 @@ void configure_hist(mb::DevState &s, const mbh_dataset *ds, int B, int kind, Run
     s.scan_grid = std::min(s.kmax * ds->F, 4 * ds->n_cu);
     s.part_launch = std::min<int32_t>(s.part_grid, 8 * ds->n_cu);
     s.part_target = 2 * ds->n_cu;
+    s.expand_slices = s.n_tiles * ((s.tile_f + mb::kSliceF - 1) / mb::kSliceF);
+    s.expand = allow_expand && ds->n <= kExpandRows && s.expand_slices <= kExpandSlices ? 1 : 0;
+    if (s.expand) {
+        // two blocks per CU over the slices; a partial per partition task
+        s.part_grid = (int32_t)((ds->n + mb::kExpandChunkMin - 1) / mb::kExpandChunkMin + s.kmax);
+        s.part_target = std::max(1, 2 * ds->n_cu / s.expand_slices);
+        s.part_launch = std::min<int32_t>(s.part_grid, s.part_target);
+        s.pb_grid = s.part_grid;
+    }
     // the root's batch gets the launch of larger tasks only where its rows
     // fill them (C2's 10.5M: 16K-row tasks; C5's 2M rows would leave three
     // quarters of each task's slots empty)
@@ -664,7 +680,8 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
     s.e_cap = 1 + 2 * max_exp;
     if (quantized) s.hist = dalloc<int32_t>((size_t)(1 + max_exp) * F * ds->nb * 3, run.arena);
     else s.histf = dalloc<mb::HistF>((size_t)(1 + max_exp) * F * ds->nb, run.arena);
-    configure_hist(s, ds, quantized ? p->num_grad_quant_bins : 4, kind, run);
+    configure_hist(s, ds, quantized ? p->num_grad_quant_bins : 4, kind, !p->time_histograms && p->partition_mode != 1,
+                   run);
     if (wide) {
         if (!stage16) s.gq = dalloc<int32_t>(2 * (size_t)ds->n, run.arena);
         s.magpart = dalloc<float>(2 * 256, run.arena);
@@ -1002,7 +1019,7 @@ mb::DevState clone_class_state(const mb::DevState &s0, const mbh_dataset *ds, in
     s.part_c = nullptr;
     s.fpart_g = s.fpart_h = nullptr;
     s.fpart_c = nullptr;
-    configure_hist(s, ds, s0.hp.quantized ? s0.hp.quant_bins : 4, kind, run);
+    configure_hist(s, ds, s0.hp.quantized ? s0.hp.quant_bins : 4, kind, s0.expand != 0, run);
     if (s0.gq) s.gq = dalloc<int32_t>(2 * (size_t)n, run.arena);
     if (s0.magpart) s.magpart = dalloc<float>(2 * 256, run.arena);
     if (s0.stage16_over) {

@@ -2818,11 +2818,12 @@ __global__ __launch_bounds__(kPartRecThreads) void k_partition_rec(DevState s) {
 template <class Acc>
 __host__ __device__ constexpr size_t slice_bytes(int ls) {
     return std::is_same<Acc, FAcc>::value ? (size_t)16 * kSliceF * ls + (size_t)4 * kSliceF * ((ls + 1) / 2)
+           : std::is_same<Acc, QAcc>::value ? (size_t)8 * kSliceF * ls
                                             : (size_t)12 * kSliceF * ls;
 }
 
-// A row's eight bins and its derivatives: the int16 pair in w; the int32 pair in
-// a; or both derivatives' bits (binary32 or binary64) in a, b
+// A row's eight bins and its derivatives: the int8 or int16 pair in w; the
+// int32 pair in a; or both derivatives' bits (binary32 or binary64) in a, b
 // with the GOSS weight bit in w.
 struct SliceRow {
     uint2 bins;
@@ -2835,7 +2836,9 @@ __device__ __forceinline__ void slice_load(const DevState &s, const uint8_t *rec
                                            SliceRow &o) {
     const uint8_t *p = rec + (size_t)r * s.rec_bytes;
     o.bins = *(const uint2 *)(p + off);
-    if constexpr (std::is_same<Acc, WAcc16>::value) {
+    if constexpr (std::is_same<Acc, QAcc>::value) {
+        o.w = *(const uint16_t *)(p + s.rec_bytes - 2);
+    } else if constexpr (std::is_same<Acc, WAcc16>::value) {
         o.w = *(const uint32_t *)(p + s.rec_bytes - 4);
     } else if constexpr (std::is_same<Acc, WAcc>::value) {
         const uint2 q = ((const uint2 *)s.gq)[r];
@@ -2862,7 +2865,10 @@ __device__ __forceinline__ void slice_add(const DevState &s, unsigned char *lds,
     const unsigned long long b = rot ? (v >> (8 * rot)) | (v << (64 - 8 * rot)) : v;
     unsigned long long packed = r.a;
     double g = 0.0, h = 0.0;
-    if constexpr (std::is_same<Acc, WAcc16>::value) {
+    if constexpr (std::is_same<Acc, QAcc>::value) {
+        packed = (unsigned long long)(((long long)(int8_t)(r.w & 255u) << 42) +
+                                      ((long long)(int8_t)(r.w >> 8) << 20) + 1LL);
+    } else if constexpr (std::is_same<Acc, WAcc16>::value) {
         packed = ((unsigned long long)(uint32_t)(int32_t)(int16_t)(r.w & 0xFFFFu) << 32) |
                  (uint32_t)(int32_t)(int16_t)(r.w >> 16);
     } else if constexpr (std::is_same<Acc, FAcc>::value) {
@@ -2887,7 +2893,8 @@ __device__ __forceinline__ void slice_add(const DevState &s, unsigned char *lds,
         } else {
             unsigned long long *a = (unsigned long long *)lds;
             atomicAdd(&a[bin * kSliceF + p], packed);
-            atomicAdd((uint32_t *)(a + kSliceF * ls) + bin * kSliceF + p, 1u);
+            if constexpr (!std::is_same<Acc, QAcc>::value)
+                atomicAdd((uint32_t *)(a + kSliceF * ls) + bin * kSliceF + p, 1u);
         }
     }
 }
@@ -2934,13 +2941,13 @@ __device__ __forceinline__ void slice_store(const DevState &s, const unsigned ch
             for (int i = 0; i < 4; ++i) {
                 const bool in = b + i < nb;
                 v[i] = in ? a[(b + i) * kSliceF + f] : 0ULL;
-                vc[i] = in ? cs[(b + i) * kSliceF + f] : 0u;
+                if constexpr (!std::is_same<Acc, QAcc>::value) vc[i] = in ? cs[(b + i) * kSliceF + f] : 0u;
             }
             *(ulonglong2 *)(s.part + o) = make_ulonglong2(v[0], v[1]);
-            *(uint2 *)(s.part_c + o) = make_uint2(vc[0], vc[1]);
-            if (two) {
-                *(ulonglong2 *)(s.part + o + 2) = make_ulonglong2(v[2], v[3]);
-                *(uint2 *)(s.part_c + o + 2) = make_uint2(vc[2], vc[3]);
+            if (two) *(ulonglong2 *)(s.part + o + 2) = make_ulonglong2(v[2], v[3]);
+            if constexpr (!std::is_same<Acc, QAcc>::value) {
+                *(uint2 *)(s.part_c + o) = make_uint2(vc[0], vc[1]);
+                if (two) *(uint2 *)(s.part_c + o + 2) = make_uint2(vc[2], vc[3]);
             }
         }
     }
@@ -3055,6 +3062,147 @@ __global__ __launch_bounds__(kAccThreads) void k_accum(DevState s) {
         __syncthreads();
         Acc::template store<LPR>(s, lds, blk, f0, Ft);
         __syncthreads();  // the LDS histogram is zeroed again for the next task
+    }
+}
+
+// Small data: a batch's partition and accumulation in one launch, where the
+// two launches are latency and not bytes. A task is a chunk of a leaf's parent
+// rows x a feature slice: a block loads the batch header, the items and the
+// round together, then its rows' ids, then the split feature's bins with the
+// rows' slice of bins and derivatives, routes each row in its thread, adds the
+// smaller child's rows and stores its features of the chunk's partial -- four
+// memory round trips, where the partition and the accumulation had four and
+// five. The blocks of slice 0 also write the partition's output, as k_partition
+// does. Every slice loads ids and split bins again, which small data has in
+// the caches, and adds with half its lanes (the larger child's rows idle), so
+// more rows or slices (kExpandRows, kExpandSlices) cost what the launch saves.
+// A launch against k_partition + k_accum: 2K x 9, 15 leaves, int8: 5.1 us
+// against 4.6 + 3.4; 100K x 28, 31 leaves, fp32: 16.7 against 6.2 + 11.6, and
+// more partials to merge; 300K x 50, int8, in three streams: 32 against 7.6 +
+// 13.6. An estimator's fit of 50K x 20: 38.6 -> 36.9 ms.
+constexpr int kExpandThreads = 512;
+template <class Acc>
+__global__ __launch_bounds__(kExpandThreads) void k_expand(DevState s) {
+    constexpr int R = kExpandChunk / kExpandThreads, NW = kExpandThreads / 64, E = R * NW;
+    static_assert(E <= 64 && NW >= 2, "one wave scans a side's entries");
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ int cnt_l[E], cnt_r[E];
+    __shared__ int base[2];
+    const int tid = threadIdx.x, lane = lane_id(), w = tid >> 6;
+    // items past the batch's are allocated, loaded and never used
+    PartItem pit = s.part_items[lane < s.kmax ? lane : 0];
+    const double goss_mult = s.round->goss_mult;
+    const Batch bh = *s.batch;
+    const int n_blocks = bh.n_blocks;
+    if ((int)blockIdx.x >= n_blocks) return;
+    const unsigned long long below = (1ULL << lane) - 1ULL;
+    const uint32_t n32 = (uint32_t)s.n;
+    const int per = (s.tile_f + kSliceF - 1) / kSliceF;
+    const int tile = (int)blockIdx.y / per, off = ((int)blockIdx.y - tile * per) * kSliceF;
+    const int f0 = tile * s.tile_f + off;
+    const int Ft = min(kSliceF, min(s.tile_f - off, s.n_features - f0));
+    if (Ft <= 0) return;  // the last tile may hold fewer slices; never slice 0
+    const uint8_t *rec = s.records + (size_t)tile * s.n * s.rec_bytes;
+    for (int blk = blockIdx.x; blk < n_blocks; blk += gridDim.x) {
+        const unsigned long long own = __ballot(lane < bh.n_items && pit.qoff <= blk);  // item 0 starts at 0
+        const int q = 63 - (int)__builtin_clzll(own);
+        const int begin = (int)readlane_i64(pit.begin, q);
+        const int nl = (int)readlane_i64(pit.n_left, q), m = (int)readlane_i64(pit.m, q);
+        const int c0 = (blk - __builtin_amdgcn_readlane(pit.qoff, q)) * bh.chunk_p;
+        const int c1 = c0 + bh.chunk_p < m ? c0 + bh.chunk_p : m;
+        const int src_buf = __builtin_amdgcn_readlane(pit.src_buf, q);
+        const int feature = __builtin_amdgcn_readlane(pit.feature, q);
+        const int thr = __builtin_amdgcn_readlane(pit.bin, q);
+        const int dl = __builtin_amdgcn_readlane(pit.default_left, q);
+        const int mb = __builtin_amdgcn_readlane(pit.missing_bin, q);
+        const int cat_e = __builtin_amdgcn_readlane(pit.cat_e, q);
+        const int direct = __builtin_amdgcn_readlane(pit.direct, q);
+        const int32_t *src = (src_buf ? s.rows1 : s.rows0) + begin;
+        int32_t *dst = (src_buf ? s.rows0 : s.rows1) + begin;
+        unsigned long long cset[4] = {0ULL, 0ULL, 0ULL, 0ULL};
+        const bool is_cat = cat_e >= 0;
+        if (is_cat)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) cset[j] = s.e_cat[(size_t)cat_e * 4 + j];
+        // every load unconditional: a row past the task is row 0, masked off
+        const __amdgpu_buffer_rsrc_t ids = buffer_rsrc(src + c0, (uint32_t)(c1 - c0) * 4u);
+        const __amdgpu_buffer_rsrc_t col = buffer_rsrc(s.bins_cm + (size_t)feature * s.n, n32);
+        uint32_t r[R], bin[R];
+        SliceRow row[R];
+        uint32_t vbits = 0, lbits = 0;
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            const int i = c0 + u * kExpandThreads + tid;
+            vbits |= (i < c1 ? 1u : 0u) << u;
+            r[u] = i < c1 ? (uint32_t)(begin + i) : 0u;
+            if (!direct) r[u] = __builtin_amdgcn_raw_buffer_load_b32(ids, (u * kExpandThreads + tid) * 4, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            if (r[u] >= n32) r[u] = 0;  // never taken: ids come from the row lists
+            bin[u] = __builtin_amdgcn_raw_buffer_load_b8(col, (int)r[u], 0, 0);
+            slice_load<Acc>(s, rec, off, r[u], goss_mult != 1.0, row[u]);
+        }
+        {  // while they load
+            uint32_t *z = (uint32_t *)lds;
+            for (int i = tid; i < (int)(slice_bytes<Acc>(s.lds_stride) / 4); i += kExpandThreads) z[i] = 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            const int b = (int)bin[u];
+            const unsigned long long cw = b < 64 ? cset[0] : b < 128 ? cset[1] : b < 192 ? cset[2] : cset[3];
+            const bool left = is_cat ? ((cw >> (b & 63)) & 1ULL) != 0 : (b == mb) ? (dl != 0) : (b <= thr);
+            lbits |= (left ? 1u : 0u) << u;
+        }
+        if (blockIdx.y == 0) {  // the partition's output
+#pragma unroll
+            for (int u = 0; u < R; ++u) {
+                const unsigned long long lm = __ballot((vbits >> u) & (lbits >> u) & 1u);
+                const unsigned long long rm = __ballot((vbits >> u) & ~(lbits >> u) & 1u);
+                if (lane == 0) {
+                    cnt_l[u * NW + w] = __popcll(lm);
+                    cnt_r[u * NW + w] = __popcll(rm);
+                }
+            }
+            __syncthreads();
+            if (w < 2) {  // wave 0 the left side, wave 1 the right one
+                int *c = w == 0 ? cnt_l : cnt_r;
+                const int v = lane < E ? c[lane] : 0;
+                const int inc = wave_incl_scan_i(v);
+                if (lane < E) c[lane] = inc - v;
+                if (lane == 63) {
+                    unsigned long long *cur = (unsigned long long *)&s.cursor[2 + 2 * q + w];
+                    base[w] = inc ? (int)atomicAdd(cur, (unsigned long long)inc) : 0;
+                }
+            }
+        }
+        __syncthreads();  // the histogram is zeroed
+        const uint32_t take = vbits & (nl <= m - nl ? lbits : ~lbits);  // the smaller child's rows (left on ties)
+#pragma unroll
+        for (int u = 0; u < R; ++u)
+            if ((take >> u) & 1u) slice_add<Acc>(s, lds, Ft, goss_mult, row[u]);
+        if (blockIdx.y == 0) {
+            // positions relative to the leaf's begin; a store past its range
+            // is dropped by the buffer and flagged
+            const int bl = base[0], br = base[1];
+            const __amdgpu_buffer_rsrc_t out = buffer_rsrc(dst, (uint32_t)m * 4u);
+            bool overflow = false;
+#pragma unroll
+            for (int u = 0; u < R; ++u) {
+                const bool valid = (vbits >> u) & 1u, left = (lbits >> u) & 1u;
+                const unsigned long long lm = __ballot(valid && left);
+                const unsigned long long rm = __ballot(valid && !left);
+                const int k = u * NW + w;
+                const int pl = bl + cnt_l[k] + (int)__popcll(lm & below);
+                const int pr = nl + br + cnt_r[k] + (int)__popcll(rm & below);
+                overflow |= valid && (left ? pl >= nl : pr >= m);
+                if (valid) __builtin_amdgcn_raw_buffer_store_b32((int)r[u], out, (left ? pl : pr) * 4, 0, 0);
+            }
+            if (overflow) atomicOr(s.error, 1);
+        }
+        __syncthreads();
+        slice_store<Acc>(s, lds, blk, f0, Ft);
+        __syncthreads();  // the LDS is the next task's
     }
 }
 
@@ -5464,14 +5612,18 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
         int64_t chunk = (built_total + s.pb_launch - 1) / s.pb_launch;
         if (chunk < s.hist_chunk_min) chunk = s.hist_chunk_min;
         if (chunk > s.hist_chunk_limit) chunk = s.hist_chunk_limit;
-        const int pc = lane < nsel ? (int)((mb + chunk - 1) / chunk) : 0;
         long long chunk_p = (rows_total + s.part_target - 1) / s.part_target;
         chunk_p = (chunk_p + kPartChunkStep - 1) / kPartChunkStep * kPartChunkStep;
         // the root's batch has a launch of its own with larger tasks
         const long long cmax = s.rcp ? (long long)kPartRecThreads * kPartRows
-                               : root_mode && s.part_root ? kPartChunkRoot : kPartChunk;
-        chunk_p = chunk_p < kPartChunkMin ? kPartChunkMin : chunk_p > cmax ? cmax : chunk_p;
+                               : s.expand                 ? kExpandChunk
+                               : root_mode && s.part_root ? kPartChunkRoot
+                                                          : kPartChunk;
+        const long long cmin = s.expand ? kExpandChunkMin : kPartChunkMin;
+        chunk_p = chunk_p < cmin ? cmin : chunk_p > cmax ? cmax : chunk_p;
         const int qc = lane < nsel ? (int)((m + chunk_p - 1) / chunk_p) : 0;
+        // k_expand: a partition task leaves the partial of its own rows
+        const int pc = s.expand ? qc : lane < nsel ? (int)((mb + chunk - 1) / chunk) : 0;
         const int pi = wave_incl_scan_i(pc), qi = wave_incl_scan_i(qc);
         if (lane < nsel) {
             v.pcnt[lane] = (int)pc;
@@ -6257,7 +6409,20 @@ hipError_t launch_hist(const DevState &s, hipStream_t st, hipEvent_t ev0, hipEve
            : s.hp.quantized ? launch_hist_t<QAcc>(s, st, ev0, ev1)
                             : launch_hist_t<FAcc>(s, st, ev0, ev1);
 }
+template <class Acc>
+hipError_t launch_expand_t(const DevState &s, hipStream_t st) {
+    hipLaunchKernelGGL(k_expand<Acc>, dim3(s.part_launch, s.expand_slices), dim3(kExpandThreads),
+                       slice_bytes<Acc>(s.lds_stride), st, s);
+    return hipGetLastError();
+}
+hipError_t launch_expand(const DevState &s, hipStream_t st) {
+    return s.hp.stage16     ? launch_expand_t<WAcc16>(s, st)
+           : s.hp.wide      ? launch_expand_t<WAcc>(s, st)
+           : s.hp.quantized ? launch_expand_t<QAcc>(s, st)
+                            : launch_expand_t<FAcc>(s, st);
+}
 hipError_t launch_partition(const DevState &s, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1, bool root) {
+    if (s.expand) return launch_expand(s, st);
     if (s.rcp) {
         // a CU holds several record-partition blocks: the grid is widened
         // to keep the same rows in flight
@@ -6285,6 +6450,7 @@ hipError_t launch_accum_t(const DevState &s, hipStream_t st, hipEvent_t ev0, hip
     }
 }
 hipError_t launch_accum(const DevState &s, hipStream_t st, hipEvent_t ev0, hipEvent_t ev1) {
+    if (s.expand) return hipSuccess;  // launch_partition's kernel accumulated
     if (s.rcp) {
         const size_t lds = hist_lds_bytes(s);
         const dim3 grid(s.pb_launch), block(kAccThreads);

@@ -144,6 +144,11 @@ constexpr int kPartChunkMin = MB_PART_CHUNK_MIN;
 constexpr int kPartChunkStep = 256;
 // Features of a slice of an accumulation task (small batches, k_accum).
 constexpr int kSliceF = 8;
+// Small data (DevState.expand): one launch partitions a batch and accumulates
+// the smaller children, in tasks of kExpandChunkMin..kExpandChunk parent rows
+// times slices of kSliceF features.
+constexpr int kExpandChunkMin = 1024;
+constexpr int kExpandChunk = 2048;
 // Rows one fp32-path histogram block may add: its counts are 16-bit halves
 // of 32-bit LDS cells.
 constexpr int64_t kFAccChunk = 65535;
@@ -402,6 +407,10 @@ struct DevState {
     int32_t hist_slices;   // slices of the root build (1: none)
     int32_t part_launch;   // blocks of a partition launch (grid-strided)
     int32_t part_target;   // partition tasks a batch is spread over
+    // 1: k_expand runs a batch (partition and accumulation in one launch,
+    // expand_slices feature slices), 0: k_partition, then k_accum
+    int32_t expand;
+    int32_t expand_slices;
     int32_t part_root;     // 1: the root's batch takes its own launch of kPartChunkRoot-row tasks
     // tree being grown (max 2 * num_leaves - 1 nodes)
     int32_t *t_feature, *t_threshold, *t_left, *t_right, *t_default_left, *t_missing_bin;

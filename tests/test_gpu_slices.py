@@ -56,3 +56,33 @@ def test_slice_training(n, f, kw):
     assert np.max(np.abs(fit.train_raw() - want)) <= 1e-5 * np.max(np.abs(want))
     for k in ("feature", "threshold", "left", "right"):
         assert np.array_equal(getattr(fit, k), getattr(ref, k)), k
+
+
+@pytest.mark.parametrize("n,f,nb,kw", [
+    (1, 1, 4, dict(min_data_in_leaf=1)),
+    (1_023, 8, 256, {}), (1_025, 9, 63, {}),           # chunks and slices of one launch
+    (65_536, 20, 255, {}), (65_537, 20, 255, {}),      # the last rows of one launch, the first of two
+    (20_000, 48, 33, {}), (20_000, 49, 33, {}),        # the most slices, and one more
+    (30_000, 12, 64, dict(quant_scale_rule=1, bagging_fraction=0.7, bagging_freq=1)),
+    (30_000, 12, 64, dict(goss=1, top_rate=0.2, other_rate=0.2, learning_rate=0.5)),
+    (9_000, 6, 40, dict(num_leaves=255, min_data_in_leaf=2)),
+])
+def test_one_launch_expansion(n, f, nb, kw):
+    """Quantized trees of small data, where one launch partitions and
+    accumulates: the CPU oracle's, bit for bit, missing bins among them."""
+    from mojoboost_amd import device
+
+    rng = np.random.default_rng(n + f)
+    bins = rng.integers(0, nb, size=(f, n)).astype(np.uint8)
+    missing = np.where(np.arange(f) % 3 == 0, nb - 1, -1).astype(np.int32)
+    z = bins[0] / nb + (bins[-1] / nb) ** 2 + 0.4 * rng.normal(size=n)
+    y = (z > np.median(z)).astype(np.float64)
+    p = dict(objective=1, num_iterations=5, num_leaves=20, min_data_in_leaf=10, lambda_l2=1.0, learning_rate=0.1)
+    p.update(kw)
+    fit = device.Dataset(bins, n, f, nb, y, missing_bin=missing).train(**p)
+    ref = O.train(bins.ravel(), n, f, nb, y, O.default_params(**p, use_quantized_grad=1), missing_bin=missing)
+    assert fit.n_trees == ref.n_trees
+    for k in ("feature", "threshold", "left", "right", "default_left"):
+        assert np.array_equal(getattr(fit, k), getattr(ref, k)), k
+    for k in ("value", "gain", "count"):
+        assert np.array_equal(getattr(fit, k).view(np.uint64), getattr(ref, k).view(np.uint64)), k
