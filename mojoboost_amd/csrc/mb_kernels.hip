@@ -3292,7 +3292,8 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan(DevState s, int root_m
     if ((int)blockIdx.x >= n_tasks) return;
     const Round rd = *s.round;
     if (rd.stopped) return;
-    const double gu = rd.grad_units, hu = rd.hess_units;
+    const double hu = rd.hess_units;
+    const QUnits qu = q_units(rd.grad_units, hu);
     const double l1 = hp.lambda_l1, l2 = hp.lambda_l2;
     long long hmin = 0;  // hessian_units_at_least: min_sum_hessian in lattice units, rounded up
     if (hp.min_sum_hessian > 0.0) {
@@ -3479,14 +3480,14 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan(DevState s, int root_m
                                                                       : ncf + 1 <= hp.max_cat_to_onehot);
         bool cat_sorted = false;
         if (ncf > 0) {
-            const double parent = qscore(TG, TH, gu, hu, l1, l2);
+            const double parent = qscore(TG, TH, qu, l1, l2);
             const long long min_c = hp.min_data_in_leaf;
             if (cat_onehot) {
                 // _onehot_search (:478-525): each category alone goes left;
                 // the argmax below keeps the lowest bin on equal gains
                 if (!gated && ncf >= 2 && bin >= 1 && bin <= ncf && !(vc < min_c || vh < hmin) &&
                     !(TC - vc < min_c) && !(TH - vh < hmin)) {
-                    const double gain = qscore(vg, vh, gu, hu, l1, l2) + qscore(TG - vg, TH - vh, gu, hu, l1, l2) - parent;
+                    const double gain = qscore(vg, vh, qu, l1, l2) + qscore(TG - vg, TH - vh, qu, l1, l2) - parent;
                     if (gain > best_gain) {
                         best_gain = gain;
                         best_order = bin;
@@ -3500,7 +3501,8 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan(DevState s, int root_m
                 // walked from both ends
                 cat_sorted = true;
                 const bool cand = !gated && ncf >= 2 && bin >= 1 && bin <= ncf && (double)vc >= hp.cat_smooth;
-                const double key = ((double)vg / gu) / ((double)vh / hu + hp.cat_smooth);
+                const double key =
+                    div_by((double)vg, qu.gu, qu.rg) / (div_by((double)vh, qu.hu, qu.rh) + hp.cat_smooth);
                 ckey[child][bin] = cand ? key : 0.0;
                 const unsigned long long cm = __ballot(cand);
                 if (lane == 0) cwcnt[wv] = __popcll(cm);
@@ -3612,7 +3614,7 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan(DevState s, int root_m
                             double bg = 0.0;
                             int bo = 0x7FFFFFFF;
                             if (mev) {
-                                const double g_ = qscore(mg, mh, gu, hu, l1, l2c) + qscore(TG - mg, TH - mh, gu, hu, l1, l2c) - parent;
+                                const double g_ = qscore(mg, mh, qu, l1, l2c) + qscore(TG - mg, TH - mh, qu, l1, l2c) - parent;
                                 if (g_ > 0.0) {
                                     bg = g_;
                                     bo = i;
@@ -3644,13 +3646,13 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan(DevState s, int root_m
             int lim = n_scan < s.widths[f] ? n_scan : s.widths[f];
             if (mc == 0 && lim > n_scan - 1) lim = n_scan - 1;
             if (bin < lim) {
-                const double parent = qscore(TG, TH, gu, hu, l1, l2);
+                const double parent = qscore(TG, TH, qu, l1, l2);
                 if (mbf >= 0) {
                     const int ag = lg + mg, ah = lh + mh, ac = lc + mc;
                     const int rg = TG - ag, rh = TH - ah, rc = TC - ac;
                     if (!(ah < hmin || rh < hmin || ac < min_c || rc < min_c)) {
                         const double gain =
-                            qscore(ag, ah, gu, hu, l1, l2) + qscore(rg, rh, gu, hu, l1, l2) - parent;
+                            qscore(ag, ah, qu, l1, l2) + qscore(rg, rh, qu, l1, l2) - parent;
                         if (gain > best_gain) {
                             best_gain = gain;
                             best_order = 2 * bin;
@@ -3662,7 +3664,7 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan(DevState s, int root_m
                     const int rg = TG - lg, rh = TH - lh, rc = TC - lc;
                     if (!(lh < hmin || rh < hmin || lc < min_c || rc < min_c)) {
                         const double gain =
-                            qscore(lg, lh, gu, hu, l1, l2) + qscore(rg, rh, gu, hu, l1, l2) - parent;
+                            qscore(lg, lh, qu, l1, l2) + qscore(rg, rh, qu, l1, l2) - parent;
                         if (gain > best_gain) {
                             best_gain = gain;
                             best_order = 2 * bin + 1;
@@ -3806,7 +3808,8 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan_narrow(DevState s, int
     if ((int)blockIdx.x >= n_tasks) return;
     const Round rd = *s.round;
     if (rd.stopped) return;
-    const double gu = rd.grad_units, hu = rd.hess_units;
+    const double hu = rd.hess_units;
+    const QUnits qu = q_units(rd.grad_units, hu);
     const double l1 = hp.lambda_l1, l2 = hp.lambda_l2;
     long long hmin = 0;  // hessian_units_at_least: min_sum_hessian in lattice units, rounded up
     if (hp.min_sum_hessian > 0.0) {
@@ -3984,13 +3987,13 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan_narrow(DevState s, int
                 int lim = n_scan < fwidth ? n_scan : fwidth;
                 if (mc == 0 && lim > n_scan - 1) lim = n_scan - 1;
                 if (bin < lim) {
-                    const double parent = qscore(TG, TH, gu, hu, l1, l2);
+                    const double parent = qscore(TG, TH, qu, l1, l2);
                     if (mbf >= 0) {
                         const int ag = lg + mg, ah = lh + mh, ac = lc + mc;
                         const int rg = TG - ag, rh = TH - ah, rc = TC - ac;
                         if (!(ah < hmin || rh < hmin || ac < min_c || rc < min_c)) {
                             const double gain =
-                                qscore(ag, ah, gu, hu, l1, l2) + qscore(rg, rh, gu, hu, l1, l2) - parent;
+                                qscore(ag, ah, qu, l1, l2) + qscore(rg, rh, qu, l1, l2) - parent;
                             if (gain > best_gain) {
                                 best_gain = gain;
                                 best_order = 2 * bin;
@@ -4002,7 +4005,7 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan_narrow(DevState s, int
                         const int rg = TG - lg, rh = TH - lh, rc = TC - lc;
                         if (!(lh < hmin || rh < hmin || lc < min_c || rc < min_c)) {
                             const double gain =
-                                qscore(lg, lh, gu, hu, l1, l2) + qscore(rg, rh, gu, hu, l1, l2) - parent;
+                                qscore(lg, lh, qu, l1, l2) + qscore(rg, rh, qu, l1, l2) - parent;
                             if (gain > best_gain) {
                                 best_gain = gain;
                                 best_order = 2 * bin + 1;
