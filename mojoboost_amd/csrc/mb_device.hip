@@ -1286,7 +1286,9 @@ int32_t mbh_train(mbh_dataset *ds, const mbh_params *p, mbh_fit **out, char *err
         fit->base = base_scores_for(ds, p->objective, K);
         double *d_base = dalloc<double>(K, run.arena);
         HIPX(hipMemcpy(d_base, fit->base.data(), K * sizeof(double), hipMemcpyHostToDevice));
-        const int grid_rows = 8 * ds->n_cu;
+        // no more blocks than have a row (2K rows: k_objective 13 us over 2048
+        // blocks, 8 have one)
+        const int grid_rows = (int)std::min<int64_t>(8 * (int64_t)ds->n_cu, (ds->n + 255) / 256);
         HIPX(mb::launch_fill_f64(s.raw, ds->n, K, d_base, grid_rows, nullptr));
         HIPX(mb::prepare_kernels(s));
         const int grid_score = mb::rows_grid(s, mb::kRowsScore, ds->n_cu);
@@ -1390,7 +1392,7 @@ int32_t mbh_train(mbh_dataset *ds, const mbh_params *p, mbh_fit **out, char *err
                 if (z.hp.goss && z.hp.quantized) HIPX(mb::launch_goss_stats(z, grid_rows, c.st));
                 if (z.hp.wide) HIPX(mb::launch_magnitude(z, c.st));
                 const bool fuse_q = mb::acc_kind(z.hp) == mb::kAccQuant && !z.hp.grad64;
-                const bool q_rows = !fuse_q || z.hp.bagging || z.hp.goss;
+                const bool q_rows = (z.hp.quantized && !fuse_q) || z.hp.bagging || z.hp.goss;
                 HIPX(mb::launch_quantize(z, q_rows ? grid_rows : 1, c.st, !fuse_q));
                 HIPX(mb::launch_hist(z, c.st, nullptr, nullptr, fuse_q));
                 HIPX(mb::launch_scan(z, 1, c.st));
@@ -1471,9 +1473,10 @@ int32_t mbh_train(mbh_dataset *ds, const mbh_params *p, mbh_fit **out, char *err
             // the max-abs lattice quantizes in the root build, which reads
             // every record of the round's rows anyway
             const bool fuse_q = mb::acc_kind(s.hp) == mb::kAccQuant && !s.hp.grad64;
-            // with the pairs written by the root build and no row list to
-            // gather (no bag, no GOSS), one block publishes the scales
-            const bool q_rows = !fuse_q || s.hp.bagging || s.hp.goss;
+            // with the pairs written by the root build (or none: binary32
+            // derivatives) and no row list to gather (no bag, no GOSS), one
+            // block publishes the scales
+            const bool q_rows = (s.hp.quantized && !fuse_q) || s.hp.bagging || s.hp.goss;
             // ... in the previous tree's round-end launch when nothing is
             // launched between the two
             const bool merge_rq = K == 1 && fuse_objective && !s.hp.goss && !s.hp.wide && !q_rows;

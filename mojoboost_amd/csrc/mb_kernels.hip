@@ -27,6 +27,8 @@
 // quantized_split_gain, tree.grow_tree_leaves_profiled and
 // growth_policy.GrowthSchedule.next_leaf (leaf choice), and
 // boosting._add_by_leaf (score update).
+#include <algorithm>
+
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
@@ -6520,7 +6522,8 @@ int rows_grid(const DevState &s, RowsKernel k, int n_cu) {
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 256, lds) != hipSuccess) per_cu = 8;
     per_cu = per_cu < 1 ? 1 : per_cu > 8 ? 8 : per_cu;
-    return per_cu * (n_cu < 1 ? 1 : n_cu);
+    // a row per thread where there are that few
+    return (int)std::min<int64_t>((int64_t)per_cu * (n_cu < 1 ? 1 : n_cu), (s.n + 255) / 256);
 }
 hipError_t launch_round_combine(const RoundStates &rs, int sampling, hipStream_t st) {
     hipLaunchKernelGGL(k_round_combine, dim3(1), dim3(64), 0, st, rs, sampling);
