@@ -4986,7 +4986,7 @@ __device__ __forceinline__ void publish_header(Batch *host, const Batch &b) {
 __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode, Batch *host) {
     extern __shared__ unsigned char plan_smem[];
     __shared__ Grow g;
-    __shared__ int s_nc, s_done, s_ncand, s_nsel, s_total, s_x, s_vf;
+    __shared__ int s_nc, s_done, s_ncand, s_nsel, s_total, s_x;
     __shared__ unsigned long long s_rows_built, s_rows_parted;
     __shared__ long long s_chunk, s_chunk_p;
     __shared__ int s_total_p;
@@ -4994,57 +4994,66 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
     const int nthr = blockDim.x, nwaves = blockDim.x >> 6;
     const int L = s.hp.num_leaves, F = s.n_features;
     const HyperParams &hp = s.hp;
-    // When the explored nodes, the frontier, the features and the items fit
-    // one per thread, every array the set-up needs is read up to its
-    // capacity first, with the batch header below in flight at the same
-    // time: one memory round trip instead of two (entries past the header's
-    // counts are allocated, read and never used).
+    // Every array the set-up needs is read up to its capacity (of the explored
+    // nodes, the first entry of each thread) with the batch header below in
+    // flight at the same time: one memory round trip instead of two (entries
+    // past the header's counts are allocated, read and never used).
     constexpr int kPW = 8;  // fold: pairs per wave (16 waves x 8 >= 2 x 64)
     static_assert(kPlanThreads / 64 * kPW >= 2 * 64, "every pair of a batch in one pass");
-    const bool pre = s.e_cap <= kPlanThreads && L <= kPlanThreads;  // launch-uniform
     const bool folded = F > 64;  // k_fold left one (gain, feature) per pair
+    const int wvu = __builtin_amdgcn_readfirstlane(wv);
     double p_eg = 0.0, gq[kPW], p_pg = 0.0;
-    int p_pf = 0x7FFFFFFF;
+    int bq[kPW], p_pf = 0x7FFFFFFF, p_bl = 0;
     int p_el = 0, p_ep = 0, p_rw = 0, p_se = 0, p_sf = 0, p_mb = 0;
     static_assert(sizeof(Item) == 64, "an item is four 16-byte words");
     uint4 p_i0 = make_uint4(0, 0, 0, 0), p_i1 = p_i0, p_i2 = p_i0, p_i3 = p_i0;
-    if (pre) {
-        if (tid < s.e_cap) {
-            p_eg = s.e_gain[tid];
-            p_el = s.e_left[tid];
-            p_ep = s.e_parent[tid];
-            p_rw = s.e_rows[tid];
-        }
-        if (tid < L) {
-            p_se = s.slot_e[tid];
-            p_sf = s.slot_fid[tid];
-        }
-        if (tid < F) p_mb = s.missing_bin[tid];
-        if (tid < s.kmax) {
-            const uint4 *q = (const uint4 *)&s.items[tid];
-            p_i0 = q[0];
-            p_i1 = q[1];
-            p_i2 = q[2];
-            p_i3 = q[3];
-        }
-        if (!folded) {
+    // The fold reads the dense gains (scan_gain: the gain of a found split,
+    // else -1), 8 bytes per (pair, feature): the planner's one CU moves a
+    // few lines per wave load instead of a line per lane. Every load
+    // unconditional (a branch between dependent loads would cost a memory
+    // round trip each): when F <= 64 wave w takes pairs w + 16 k, k < kPW,
+    // lane = feature; the argmax keeps the lowest feature on equal gains.
+    // With more features k_fold has already folded each pair (same rule),
+    // and thread p reads pair p's (gain, feature).
+    if (!folded) {
 #pragma unroll
-            for (int k = 0; k < kPW; ++k) {
-                int pr = wv + k * nwaves;
-                pr = pr < 2 * s.kmax ? pr : 0;
-                gq[k] = s.scan_gain[(size_t)pr * F + (lane < F ? lane : 0)];
-            }
-        } else if (tid < 2 * s.kmax) {
-            p_pg = s.pair_gain[tid];
-            p_pf = s.pair_feat[tid];
+        for (int k = 0; k < kPW; ++k) {
+            int pr = wvu + k * nwaves;
+            pr = pr < 2 * s.kmax ? pr : 0;
+            gq[k] = s.scan_gain[(size_t)pr * F + (lane < F ? lane : 0)];
+            bq[k] = s.items[pr >> 1].builds_left;
         }
+    } else if (tid < 2 * s.kmax) {
+        p_pg = s.pair_gain[tid];
+        p_pf = s.pair_feat[tid];
+        p_bl = s.items[tid >> 1].builds_left;
     }
-    // the batch size, the round and the growth counters in one memory round
+    if (tid < s.e_cap) {
+        p_eg = s.e_gain[tid];
+        p_el = s.e_left[tid];
+        p_ep = s.e_parent[tid];
+        p_rw = s.e_rows[tid];
+    }
+    if (tid < L) {  // L <= kPlanThreads
+        p_se = s.slot_e[tid];
+        p_sf = s.slot_fid[tid];
+    }
+    if (tid < F) p_mb = s.missing_bin[tid];
+    if (tid < s.kmax) {
+        const uint4 *q = (const uint4 *)&s.items[tid];
+        p_i0 = q[0];
+        p_i1 = q[1];
+        p_i2 = q[2];
+        p_i3 = q[3];
+    }
+    // the batch size, the round and the growth counters in the same round
     // trip (every thread reads the counters itself, a broadcast load, instead
     // of waiting at a barrier for one thread's copy)
     const int n_items = root_mode ? 1 : s.batch->n_items;
     const Round rd = *s.round;
-    const int ne = root_mode ? 1 : s.grow->n_explored, nl0 = root_mode ? 1 : s.grow->n_leaves;
+    Grow g0 = *s.grow;
+    if (root_mode) g0 = Grow{1, 1, 1, 1, 0, 0, 0, 0};
+    const int ne = g0.n_explored, nl0 = g0.n_leaves;
     if (n_items <= 0) {  // the tree is complete
         if (host != nullptr && tid == 0) publish_header(host, *s.batch);
         return;
@@ -5070,102 +5079,51 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
     }
     const double gu = rd.grad_units, hu = rd.hess_units;
     if (tid == 0) {
-        if (root_mode) {
-            g.n_leaves = 1;
-            g.n_nodes = 1;
-            g.n_explored = 1;
-            g.n_hist = 1;
-            g.expansions = 0;
-            g.iterations = 0;
-            g.rows_built = 0;
-            g.rows_parted = 0;
-        } else {
-            g = *s.grow;
-        }
+        g = g0;
         s_rows_built = 0;
         s_rows_parted = 0;
         s_ncand = 0;
     }
     // ---- 1. fold (one wave per pair over the pair's per-feature results).
-    // The fold's gains, the items, the explored nodes and the frontier are
-    // all loaded in one memory round trip, the gains first.
+    // Pair p's node is one of the last n_pairs explored (children follow their
+    // batch's order), the left child first.
     const int n_pairs = root_mode ? 1 : 2 * n_items;
-    // The fold reads the dense gains (scan_gain: the gain of a found split,
-    // else -1), 8 bytes per (pair, feature): the planner's one CU moves a
-    // few lines per wave load instead of a line per lane. Every load
-    // unconditional (a branch between dependent loads would cost a memory
-    // round trip each): when F <= 64 wave w takes pairs w + 16 k, k < kPW,
-    // lane = feature; the argmax keeps the lowest feature on equal gains.
-    // With more features k_fold has already folded each pair (same rule),
-    // and thread p reads pair p's (gain, feature).
-    if (pre) {
-        if (!root_mode && tid < n_items) {
-            uint4 *q = (uint4 *)&v.it[tid];
-            q[0] = p_i0;
-            q[1] = p_i1;
-            q[2] = p_i2;
-            q[3] = p_i3;
-        }
-        if (tid < F) v.mbin[tid] = p_mb;
-        for (int f = tid + nthr; f < F; f += nthr) v.mbin[f] = s.missing_bin[f];  // F > kPlanThreads
-        if (tid < ne) {
-            v.eg[tid] = p_eg;
-            v.el[tid] = p_el;
-            v.ep[tid] = p_ep;
-            v.rw[tid] = p_rw;
-        }
-        if (!root_mode && tid < nl0) {
-            v.sl_e[tid] = p_se;
-            v.sl_fid[tid] = p_sf;
-        }
-    } else {
-        if (folded) {
-            if (tid < n_pairs) {
-                p_pg = s.pair_gain[tid];
-                p_pf = s.pair_feat[tid];
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < kPW; ++k) {
-                int pr = wv + k * nwaves;
-                pr = pr < n_pairs ? pr : 0;
-                gq[k] = s.scan_gain[(size_t)pr * F + (lane < F ? lane : 0)];
-            }
-        }
-        if (!root_mode)
-            for (int jj = tid; jj < n_items; jj += nthr) v.it[jj] = s.items[jj];
-        for (int f = tid; f < F; f += nthr) v.mbin[f] = s.missing_bin[f];
-        for (int i = tid; i < ne; i += nthr) {
-            v.eg[i] = s.e_gain[i];
-            v.el[i] = s.e_left[i];
-            v.ep[i] = s.e_parent[i];
-            v.rw[i] = s.e_rows[i];
-        }
-        if (!root_mode)
-            for (int i = tid; i < nl0; i += nthr) {
-                v.sl_e[i] = s.slot_e[i];
-                v.sl_fid[i] = s.slot_fid[i];
-            }
+    const int ne_old = ne - n_pairs;
+    auto pair_node = [&](int pr, int builds_left) {
+        if (root_mode) return 0;
+        const bool built = (pr & 1) == 0;
+        return ne_old + (pr & ~1) + (built == (builds_left != 0) ? 0 : 1);
+    };
+    if (!root_mode && tid < n_items) {
+        uint4 *q = (uint4 *)&v.it[tid];
+        q[0] = p_i0;
+        q[1] = p_i1;
+        q[2] = p_i2;
+        q[3] = p_i3;
     }
-    if (hp.quantized) {
-        if (tid == 0) s_vf = 0;  // unused: integer sums give the leaf values
-    } else if (tid < 64) {
-        // the tree's first selected feature (the fp32 path's leaf value sums)
-        int vf = F - 1;
-        for (int f0 = 0; f0 < F; f0 += 64) {
-            const unsigned long long m =
-                __ballot(f0 + lane < F && s.feature_mask[(size_t)rd.tree_index * F + f0 + lane]);
-            if (m) {
-                vf = f0 + (int)__builtin_ctzll(m);
-                break;
-            }
-        }
-        if (lane == 0) s_vf = vf;
+    if (tid < F) v.mbin[tid] = p_mb;
+    for (int f = tid + nthr; f < F; f += nthr) v.mbin[f] = s.missing_bin[f];  // F > kPlanThreads
+    if (tid < ne_old) v.eg[tid] = p_eg;  // the pairs' nodes: by the fold
+    if (tid < ne) {
+        v.el[tid] = root_mode ? -1 : p_el;
+        v.ep[tid] = root_mode ? -1 : p_ep;
+        v.rw[tid] = p_rw;  // the root's: with its result below
+    }
+    for (int i = tid + nthr; i < ne; i += nthr) {  // more nodes than threads
+        if (i < ne_old) v.eg[i] = s.e_gain[i];
+        v.el[i] = s.e_left[i];
+        v.ep[i] = s.e_parent[i];
+        v.rw[i] = s.e_rows[i];
+    }
+    if (tid < nl0) {
+        v.sl_e[tid] = root_mode ? 0 : p_se;
+        v.sl_fid[tid] = root_mode ? 0 : p_sf;
     }
     if (folded) {
         if (tid < n_pairs) {
             v.wg[tid] = p_pg;
             v.wf[tid] = p_pf;
+            v.eg[pair_node(tid, p_bl)] = p_pf != 0x7FFFFFFF ? p_pg : -1.0;  // a found split has gain > 0
         }
     } else {  // F <= 64
         // Bound by the instructions of 16 waves on one CU: a maximum of the
@@ -5183,14 +5141,16 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
             }
 #pragma unroll
             for (int k = K0; k < K1; ++k) {
-                const int pr = wv + k * nwaves;
+                const int pr = wvu + k * nwaves;
                 if (pr >= n_pairs) break;  // wave-uniform
+                const int e_id = pair_node(pr, bq[k]);
                 const unsigned long long at =
                     __ballot((unsigned)((unsigned long long)__double_as_longlong(gq[k]) >> 32) == mh[k - K0]);
                 if (mh[k - K0] != 0u && (at & (at - 1ULL)) == 0ULL) {
                     if ((at >> lane) & 1ULL) {
                         v.wg[pr] = gq[k];
                         v.wf[pr] = lane;
+                        v.eg[e_id] = gq[k];
                     }
                     continue;
                 }
@@ -5200,87 +5160,14 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
                 if (lane == 0) {
                     v.wg[pr] = bg;
                     v.wf[pr] = bf;
+                    v.eg[e_id] = bf != 0x7FFFFFFF ? bg : -1.0;
                 }
             }
         };
         static_assert(kPW == 8, "the groups below");
         fold(std::integral_constant<int, 0>(), std::integral_constant<int, 1>());
-        if (wv + nwaves < n_pairs) fold(std::integral_constant<int, 1>(), std::integral_constant<int, 4>());
-        if (wv + 4 * nwaves < n_pairs) fold(std::integral_constant<int, 4>(), std::integral_constant<int, 8>());
-    }
-    __syncthreads();
-    for (int pr = tid; pr < n_pairs; pr += nthr) {
-        int e_id = 0;
-        if (!root_mode) {
-            const Item &it = v.it[pr >> 1];
-            const bool built = (pr & 1) == 0;
-            e_id = (built == (it.builds_left != 0)) ? it.left_e : it.left_e + 1;
-        }
-        const ScanResult *base = &s.scan[(size_t)pr * F];
-        const int bf = v.wf[pr];
-        const bool found = bf != 0x7FFFFFFF;
-        // the three results this pair needs, loaded together
-        const long long G = base->tot_g, H = base->tot_h, C = base->tot_c;
-        const double fg = base[s_vf].fg, fh = base[s_vf].fh;
-        const ScanResult &qb = base[found ? bf : 0];
-        const int q_bin = qb.bin, q_dl = qb.default_left, q_cat = qb.cat;
-        const long long q_nl = qb.n_left;
-        // leaf value: integer sums are the same on every feature; the fp32
-        // path sums the tree's first selected feature serially, as
-        // tree._leaf_value does (value_feature = tree_features[0])
-        const double value = hp.quantized ? qleaf(G, H, gu, hu, hp.lambda_l1, hp.lambda_l2)
-                                          : -soft_threshold_l1(fg, hp.lambda_l1) / (fh + hp.lambda_l2);
-        ENode *e = &s.enodes[e_id];
-        if (root_mode) {
-            e->begin = 0;
-            e->end = C;
-            e->buf = 0;
-            e->hist = 0;
-            e->depth = 0;
-            e->left_e = -1;
-            e->right_e = -1;
-            s.t_value[0] = value;
-            s.t_count[0] = (double)C;
-        }
-        e->tot_g = G;
-        e->tot_h = H;
-        e->tot_c = C;
-        e->value = value;
-        e->found = found ? 1 : 0;
-        e->cat = found && q_cat ? 1 : 0;
-        if (found && q_cat) {
-            const unsigned long long *sb = s.scan_cat + ((size_t)pr * F + bf) * 4;
-#pragma unroll
-            for (int w = 0; w < 4; ++w) s.e_cat[(size_t)e_id * 4 + w] = sb[w];
-        }
-        if (found) {
-            e->gain = v.wg[pr];
-            e->feature = bf;
-            e->bin = q_bin;
-            e->default_left = q_dl;
-            e->n_left = q_nl;
-        } else {
-            e->gain = 0.0;
-            e->feature = -1;
-            e->bin = -1;
-            e->default_left = 0;
-            e->n_left = 0;
-        }
-        const double eg = found ? v.wg[pr] : -1.0;  // a found split has gain > 0
-        v.eg[e_id] = eg;
-        s.e_gain[e_id] = eg;
-        if (root_mode) {
-            v.el[0] = -1;
-            v.ep[0] = -1;
-            v.rw[0] = (int32_t)C;
-            s.e_left[0] = -1;
-            s.e_parent[0] = -1;
-            s.e_rows[0] = (int32_t)C;
-        }
-    }
-    if (root_mode && tid == 0) {
-        v.sl_e[0] = 0;
-        v.sl_fid[0] = 0;
+        if (wvu + nwaves < n_pairs) fold(std::integral_constant<int, 1>(), std::integral_constant<int, 4>());
+        if (wvu + 4 * nwaves < n_pairs) fold(std::integral_constant<int, 4>(), std::integral_constant<int, 8>());
     }
     __syncthreads();
     // ---- 2. replay (wave 0), see replay_wave. Each explored node's bar (cb)
@@ -5292,7 +5179,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
     }
     __syncthreads();
     if (tid < 64) {
-        int nl = nl0, nn = g.n_nodes, nc = 0, done = 0, x = -1;
+        int nl = nl0, nn = g0.n_nodes, nc = 0, done = 0, x = -1;
         if (L <= 64) replay_wave<1>(v, L, nl, nn, nc, done, x);
         else if (L <= 256) replay_wave<4>(v, L, nl, nn, nc, done, x);
         else replay_wave<8>(v, L, nl, nn, nc, done, x);  // L <= 512: the LDS of more nodes is not there
@@ -5309,6 +5196,76 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
         for (int i = lane; i < ne; i += 64) v.fr[i] = 0;
         __asm__ volatile("" ::: "memory");
         for (int i = lane; i < nl; i += 64) v.fr[v.sl_e[i]] = 1;
+    } else if (wv <= 2) {
+        // Waves 1 and 2, beside the replay, which needs none of it: the pairs'
+        // nodes from their results, a memory round trip out of the chain
+        // (with one for the growth counters and one for the fp32 path's
+        // feature mask: 10.4 -> 9.7 us a launch at 15 leaves, 11.7 -> 10.9 at
+        // 31 leaves fp32).
+        static_assert(kPlanThreads >= 192, "a thread of waves 1 and 2 per pair");
+        // leaf value: integer sums are the same on every feature; the fp32
+        // path sums the tree's first selected feature serially, as
+        // tree._leaf_value does (value_feature = tree_features[0])
+        int vf = 0;
+        if (!hp.quantized) {
+            vf = F - 1;
+            for (int f0 = 0; f0 < F; f0 += 64) {
+                const unsigned long long m =
+                    __ballot(f0 + lane < F && s.feature_mask[(size_t)rd.tree_index * F + f0 + lane]);
+                if (m) {
+                    vf = f0 + (int)__builtin_ctzll(m);
+                    break;
+                }
+            }
+        }
+        const int pr = tid - 64;
+        if (pr < n_pairs) {
+            const int e_id = pair_node(pr, root_mode ? 0 : v.it[pr >> 1].builds_left);
+            const ScanResult *base = &s.scan[(size_t)pr * F];
+            const int bf = v.wf[pr];
+            const bool found = bf != 0x7FFFFFFF;
+            // the three results this pair needs, loaded together
+            const long long G = base->tot_g, H = base->tot_h, C = base->tot_c;
+            const double fg = base[vf].fg, fh = base[vf].fh;
+            const ScanResult &qb = base[found ? bf : 0];
+            const int q_bin = qb.bin, q_dl = qb.default_left, q_cat = qb.cat;
+            const long long q_nl = qb.n_left;
+            const double value = hp.quantized ? qleaf(G, H, gu, hu, hp.lambda_l1, hp.lambda_l2)
+                                              : -soft_threshold_l1(fg, hp.lambda_l1) / (fh + hp.lambda_l2);
+            ENode *e = &s.enodes[e_id];
+            if (root_mode) {
+                e->begin = 0;
+                e->end = C;
+                e->buf = 0;
+                e->hist = 0;
+                e->depth = 0;
+                e->left_e = -1;
+                e->right_e = -1;
+                s.t_value[0] = value;
+                s.t_count[0] = (double)C;
+                v.rw[0] = (int32_t)C;
+                s.e_left[0] = -1;
+                s.e_parent[0] = -1;
+                s.e_rows[0] = (int32_t)C;
+            }
+            e->tot_g = G;
+            e->tot_h = H;
+            e->tot_c = C;
+            e->value = value;
+            e->found = found ? 1 : 0;
+            e->cat = found && q_cat ? 1 : 0;
+            if (found && q_cat) {
+                const unsigned long long *sb = s.scan_cat + ((size_t)pr * F + bf) * 4;
+#pragma unroll
+                for (int w = 0; w < 4; ++w) s.e_cat[(size_t)e_id * 4 + w] = sb[w];
+            }
+            e->gain = found ? v.wg[pr] : 0.0;
+            e->feature = found ? bf : -1;
+            e->bin = found ? q_bin : -1;
+            e->default_left = found ? q_dl : 0;
+            e->n_left = found ? q_nl : 0;
+            s.e_gain[e_id] = v.eg[e_id];
+        }
     }
     __syncthreads();
     const int nc = s_nc, nl = g.n_leaves, nn = g.n_nodes;
@@ -5459,6 +5416,8 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
 #pragma unroll
     for (int k = 0; k < kJ; ++k) {
         const int i = tid + k * nthr;
+        myb[k] = myp[k] = -1;
+        if (k * nthr >= ne) continue;
         const bool c = i < ne && ju[k] == -1 && v.eg[i] > 0.0 && jv[k] > 0.0;
         const bool pend = c && v.el[i] < 0 && (i == s_x || v.rw[i] <= spec_rows);
         const unsigned long long m = __ballot(c), mp = __ballot(pend);
@@ -5472,7 +5431,8 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
     }
     __syncthreads();
     if (tid < 64) {
-        const int a = s_wcnt[lane], b = s_pcnt[lane];
+        const bool in = lane * 64 < ne;  // count lane is of nodes 64 lane and on
+        const int a = in ? s_wcnt[lane] : 0, b = in ? s_pcnt[lane] : 0;
         const int ia = wave_incl_scan_i(a), ib = wave_incl_scan_i(b);
         s_wcnt[lane] = ia - a;
         s_pcnt[lane] = ib - b;
@@ -5678,10 +5638,12 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
             mb = sn.n_left <= m - sn.n_left ? sn.n_left : m - sn.n_left;
         }
         const long long rows_total = wave_add_u32((unsigned)m), built_total = wave_add_u32((unsigned)mb);
-        int64_t chunk = (built_total + s.pb_launch - 1) / s.pb_launch;
+        // (and 32-bit divisions: 64-bit ones are some hundred instructions each)
+        auto ceil_div = [](long long a, long long d) { return ((unsigned)a + ((unsigned)d - 1u)) / (unsigned)d; };
+        int64_t chunk = ceil_div(built_total, s.pb_launch);
         if (chunk < s.hist_chunk_min) chunk = s.hist_chunk_min;
         if (chunk > s.hist_chunk_limit) chunk = s.hist_chunk_limit;
-        long long chunk_p = (rows_total + s.part_target - 1) / s.part_target;
+        long long chunk_p = ceil_div(rows_total, s.part_target);
         chunk_p = (chunk_p + kPartChunkStep - 1) / kPartChunkStep * kPartChunkStep;
         // the root's batch has a launch of its own with larger tasks
         const long long cmax = s.rcp ? (long long)kPartRecThreads * kPartRows
@@ -5690,9 +5652,9 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
                                                           : kPartChunk;
         const long long cmin = s.expand ? kExpandChunkMin : kPartChunkMin;
         chunk_p = chunk_p < cmin ? cmin : chunk_p > cmax ? cmax : chunk_p;
-        const int qc = lane < nsel ? (int)((m + chunk_p - 1) / chunk_p) : 0;
+        const int qc = lane < nsel ? (int)ceil_div(m, chunk_p) : 0;
         // k_expand: a partition task leaves the partial of its own rows
-        const int pc = s.expand ? qc : lane < nsel ? (int)((mb + chunk - 1) / chunk) : 0;
+        const int pc = s.expand ? qc : lane < nsel ? (int)ceil_div(mb, chunk) : 0;
         const int pi = wave_incl_scan_i(pc), qi = wave_incl_scan_i(qc);
         if (lane < nsel) {
             v.pcnt[lane] = (int)pc;
@@ -5727,7 +5689,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
         const int64_t m = e0 - b0;
         const int ebuf = sn.buf, ehist = sn.hist, edep = sn.depth;
         const bool bl = nlft <= m - nlft;
-        const int le = ne + 2 * jj, hb = g.n_hist + jj;
+        const int le = ne + 2 * jj, hb = g0.n_hist + jj;
         Item it;
         it.begin = b0;
         it.end = e0;
@@ -5743,7 +5705,6 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
         it.part_cnt = v.pcnt[jj];
         it.pad_ = 0;
         s.items[jj] = it;
-        v.it[jj] = it;
         ENode c;
         c.n_left = 0;
         c.tot_g = c.tot_h = c.tot_c = 0;
@@ -5805,8 +5766,6 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
         ai.buf = 1 - ebuf;
         s.acc_items[jj] = ai;
     }
-    __syncthreads();
-    __syncthreads();
     if (tid == 0) {
         if (s.iter_log && g.iterations < s.iter_stride) {
             int64_t *lg = s.iter_log + 2 * ((size_t)rd.tree_index * s.iter_stride + g.iterations);
