@@ -120,6 +120,28 @@ __device__ __forceinline__ float stats_max_wave(const DevState &s, int parity, i
     return __uint_as_float(wave_max_u32(s.stats[stat_slot(parity, which, lane_id())]));
 }
 
+// Keeps loads where they are written: without a use before a kernel's early
+// exit the compiler moves them behind it, a memory round trip later. For
+// kernels of few, small blocks: the partition's and the accumulation's many
+// waves lost more to loading items that an idle block never needs (10.5M x 28:
+// k_partition 35.1 -> 36.2 us, 200K x 1000: k_accum 27.6 -> 28.5 us).
+template <class T>
+__device__ __forceinline__ void loaded_v(const T &x) {  // per-lane values
+    static_assert(sizeof(T) % 4 == 0, "words");
+    uint32_t w[sizeof(T) / 4];
+    __builtin_memcpy(w, &x, sizeof(T));
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / 4; ++i) __asm__ volatile("" ::"v"(w[i]));
+}
+template <class T>
+__device__ __forceinline__ void loaded_s(const T &x) {  // wave-uniform values
+    static_assert(sizeof(T) % 4 == 0, "words");
+    uint32_t w[sizeof(T) / 4];
+    __builtin_memcpy(w, &x, sizeof(T));
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / 4; ++i) __asm__ volatile("" ::"s"(w[i]));
+}
+
 __device__ __forceinline__ unsigned wave_min_u32(unsigned x) {
     x = min(x, dpp_u32<0xB1, 0xF>(x));
     x = min(x, dpp_u32<0x4E, 0xF>(x));
@@ -3095,6 +3117,8 @@ __global__ __launch_bounds__(kExpandThreads) void k_expand(DevState s) {
     PartItem pit = s.part_items[lane < s.kmax ? lane : 0];
     const double goss_mult = s.round->goss_mult;
     const Batch bh = *s.batch;
+    loaded_s(bh);
+    loaded_v(pit);
     const int n_blocks = bh.n_blocks;
     if ((int)blockIdx.x >= n_blocks) return;
     const unsigned long long below = (1ULL << lane) - 1ULL;
@@ -3289,10 +3313,18 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan(DevState s, int root_m
     const HyperParams &hp = s.hp;
     const int F = s.n_features, nb = s.n_bins;
     const size_t hsz = (size_t)F * nb * 3;
-    const int n_items = root_mode ? 1 : s.batch->n_items;
+    // the first task's item (without scan_order) and the round load with the
+    // batch header, one memory round trip for all (15.2 -> 15.1 us a launch at
+    // 10.5M x 28, where merging bounds it)
+    const int j0 = (int)blockIdx.x / F;
+    const Item it0 = s.items[j0 < s.kmax ? j0 : 0];
+    const Round rd = *s.round;
+    const int b_items = s.batch->n_items, n_items = root_mode ? 1 : b_items;
+    loaded_s(b_items);
+    loaded_s(rd);
+    loaded_s(it0);
     const int n_tasks = n_items * F;
     if ((int)blockIdx.x >= n_tasks) return;
-    const Round rd = *s.round;
     if (rd.stopped) return;
     const double hu = rd.hess_units;
     const QUnits qu = q_units(rd.grad_units, hu);
@@ -3329,7 +3361,8 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan(DevState s, int root_m
             it.hist_sib = 0;
             it.depth_child = 0;
         } else {
-            it = s.items[j];
+            it = it0;
+            if (task != (int)blockIdx.x || (kCat && s.scan_order != nullptr)) it = s.items[j];
             const int64_t m = it.end - it.begin;
             m_built = it.builds_left ? it.n_left : m - it.n_left;
             m_sib = m - m_built;
@@ -3804,11 +3837,19 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan_narrow(DevState s, int
     const HyperParams &hp = s.hp;
     const int F = s.n_features, nb = s.n_bins;
     const size_t hsz = (size_t)F * nb * 3;
-    const int n_items = root_mode ? 1 : s.batch->n_items;
+    // every wave holds the batch's items, lane i item i (n_items <= 64): a
+    // task reads its item's fields from registers, not from memory. They and
+    // the round load with the batch header, one memory round trip (2K x 9: 4.9
+    // -> 4.6 us a launch)
+    const Item my = s.items[lane < s.kmax ? lane : 0];
+    const Round rd = *s.round;
+    const int b_items = s.batch->n_items, n_items = root_mode ? 1 : b_items;
+    loaded_s(b_items);
+    loaded_s(rd);
+    loaded_v(my);
     const int n_groups = (F + kNarrowFeat - 1) / kNarrowFeat;
     const int n_tasks = n_items * n_groups;
     if ((int)blockIdx.x >= n_tasks) return;
-    const Round rd = *s.round;
     if (rd.stopped) return;
     const double hu = rd.hess_units;
     const QUnits qu = q_units(rd.grad_units, hu);
@@ -3820,10 +3861,6 @@ __global__ __launch_bounds__(kScanThreads, 4) void k_scan_narrow(DevState s, int
         if (fl < u) fl += 1.0;
         hmin = (long long)fl;
     }
-    // every wave holds the batch's items, lane i item i (n_items <= 64): a
-    // task reads its item's fields from registers, not from memory
-    Item my{};
-    if (!root_mode && lane < n_items) my = s.items[lane];
     for (int task = blockIdx.x; task < n_tasks; task += gridDim.x) {
         const int j = task / n_groups;
         const int f0 = (task - j * n_groups) * kNarrowFeat;
@@ -4065,10 +4102,18 @@ __global__ __launch_bounds__(kScanThreads, kCat ? 1 : 4) void k_scan_f(DevState 
     const HyperParams &hp = s.hp;
     const int F = s.n_features, nb = s.n_bins;
     const size_t hsz = (size_t)F * nb;
-    const int n_items = root_mode ? 1 : s.batch->n_items;
+    // the first task's item (without scan_order) and the round load with the
+    // batch header, one memory round trip for all (100K x 28, 31 leaves: 10.5 ->
+    // 9.9 us a launch)
+    const int j0 = (int)blockIdx.x / F;
+    const Item it0 = s.items[j0 < s.kmax ? j0 : 0];
+    const Round rd = *s.round;
+    const int b_items = s.batch->n_items, n_items = root_mode ? 1 : b_items;
+    loaded_s(b_items);
+    loaded_s(rd);
+    loaded_s(it0);
     const int n_tasks = n_items * F;
     if ((int)blockIdx.x >= n_tasks) return;
-    const Round rd = *s.round;
     if (rd.stopped) return;
     const double l1 = hp.lambda_l1, l2 = hp.lambda_l2, min_h = hp.min_sum_hessian;
     const long long min_c = hp.min_data_in_leaf;
@@ -4097,7 +4142,8 @@ __global__ __launch_bounds__(kScanThreads, kCat ? 1 : 4) void k_scan_f(DevState 
             it.hist_sib = 0;
             it.depth_child = 0;
         } else {
-            it = s.items[j];
+            it = it0;
+            if (task != (int)blockIdx.x || (kCat && s.scan_order != nullptr)) it = s.items[j];
             const int64_t m = it.end - it.begin;
             m_built = it.builds_left ? it.n_left : m - it.n_left;
             m_sib = m - m_built;
@@ -4655,7 +4701,7 @@ struct SelNode {
 
 struct PlanLayout {
     size_t sn, mbin;
-    size_t wg, eg, cb, kr, wf, el, ep, rw, fr, ci, sl_e, sl_fid, cm_e, cm_fid, cm_lf, sel_e, pcnt, poff, qcnt, qoff, it;
+    size_t wg, eg, cb, kr, wf, el, ep, rw, fr, ci, sl_e, sl_fid, cm_e, cm_fid, cm_lf, sel_e, pcnt, poff, qcnt, qoff;
     size_t total;
 };
 
@@ -4688,7 +4734,6 @@ __host__ __device__ inline PlanLayout plan_layout(int L, int E, int K, int F) {
     p.poff = take((size_t)4 * (K + 1), 4);
     p.qcnt = take((size_t)4 * K, 4);
     p.qoff = take((size_t)4 * (K + 1), 4);
-    p.it = take(sizeof(Item) * K, 16);
     p.sn = take(sizeof(SelNode) * K, 16);    // the selected leaves' nodes
     p.mbin = take((size_t)4 * F, 4);         // missing bin per feature
     p.total = o;
@@ -4700,7 +4745,6 @@ struct PlanView {
     int32_t *mbin;
     double *wg, *eg, *cb, *xr;
     int32_t *wf, *el, *ep, *rw, *fr, *ci, *sl_e, *sl_fid, *cm_e, *cm_fid, *cm_lf, *sel_e, *pcnt, *poff, *qcnt, *qoff;
-    Item *it;
 };
 
 __device__ PlanView plan_view(const DevState &s, unsigned char *smem) {
@@ -4726,7 +4770,6 @@ __device__ PlanView plan_view(const DevState &s, unsigned char *smem) {
     v.poff = (int32_t *)(smem + p.poff);
     v.qcnt = (int32_t *)(smem + p.qcnt);
     v.qoff = (int32_t *)(smem + p.qoff);
-    v.it = (Item *)(smem + p.it);
     v.sn = (SelNode *)(smem + p.sn);
     v.mbin = (int32_t *)(smem + p.mbin);
     return v;
@@ -5003,10 +5046,8 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
     const bool folded = F > 64;  // k_fold left one (gain, feature) per pair
     const int wvu = __builtin_amdgcn_readfirstlane(wv);
     double p_eg = 0.0, gq[kPW], p_pg = 0.0;
-    int bq[kPW], p_pf = 0x7FFFFFFF, p_bl = 0;
+    int p_pf = 0x7FFFFFFF;
     int p_el = 0, p_ep = 0, p_rw = 0, p_se = 0, p_sf = 0, p_mb = 0;
-    static_assert(sizeof(Item) == 64, "an item is four 16-byte words");
-    uint4 p_i0 = make_uint4(0, 0, 0, 0), p_i1 = p_i0, p_i2 = p_i0, p_i3 = p_i0;
     // The fold reads the dense gains (scan_gain: the gain of a found split,
     // else -1), 8 bytes per (pair, feature): the planner's one CU moves a
     // few lines per wave load instead of a line per lane. Every load
@@ -5021,12 +5062,10 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
             int pr = wvu + k * nwaves;
             pr = pr < 2 * s.kmax ? pr : 0;
             gq[k] = s.scan_gain[(size_t)pr * F + (lane < F ? lane : 0)];
-            bq[k] = s.items[pr >> 1].builds_left;
         }
     } else if (tid < 2 * s.kmax) {
         p_pg = s.pair_gain[tid];
         p_pf = s.pair_feat[tid];
-        p_bl = s.items[tid >> 1].builds_left;
     }
     if (tid < s.e_cap) {
         p_eg = s.e_gain[tid];
@@ -5039,23 +5078,20 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
         p_sf = s.slot_fid[tid];
     }
     if (tid < F) p_mb = s.missing_bin[tid];
-    if (tid < s.kmax) {
-        const uint4 *q = (const uint4 *)&s.items[tid];
-        p_i0 = q[0];
-        p_i1 = q[1];
-        p_i2 = q[2];
-        p_i3 = q[3];
-    }
     // the batch size, the round and the growth counters in the same round
     // trip (every thread reads the counters itself, a broadcast load, instead
     // of waiting at a barrier for one thread's copy)
-    const int n_items = root_mode ? 1 : s.batch->n_items;
+    const Batch bh = *s.batch;
     const Round rd = *s.round;
     Grow g0 = *s.grow;
+    loaded_s(bh);
+    loaded_s(rd);
+    loaded_s(g0);
+    const int n_items = root_mode ? 1 : bh.n_items;
     if (root_mode) g0 = Grow{1, 1, 1, 1, 0, 0, 0, 0};
     const int ne = g0.n_explored, nl0 = g0.n_leaves;
     if (n_items <= 0) {  // the tree is complete
-        if (host != nullptr && tid == 0) publish_header(host, *s.batch);
+        if (host != nullptr && tid == 0) publish_header(host, bh);
         return;
     }
     PlanView v = plan_view(s, plan_smem);
@@ -5072,6 +5108,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
             b.n_acc = 0;
             b.chunk_p = b.chunk_a = 0;
             b.slices = 1;
+            b.left[0] = b.left[1] = 0u;
             *s.batch = b;
             if (host != nullptr) publish_header(host, b);
         }
@@ -5089,18 +5126,12 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
     // batch's order), the left child first.
     const int n_pairs = root_mode ? 1 : 2 * n_items;
     const int ne_old = ne - n_pairs;
-    auto pair_node = [&](int pr, int builds_left) {
+    const unsigned long long left = ((unsigned long long)bh.left[1] << 32) | bh.left[0];
+    auto pair_node = [&](int pr) {
         if (root_mode) return 0;
         const bool built = (pr & 1) == 0;
-        return ne_old + (pr & ~1) + (built == (builds_left != 0) ? 0 : 1);
+        return ne_old + (pr & ~1) + (built == (((left >> (pr >> 1)) & 1ULL) != 0) ? 0 : 1);
     };
-    if (!root_mode && tid < n_items) {
-        uint4 *q = (uint4 *)&v.it[tid];
-        q[0] = p_i0;
-        q[1] = p_i1;
-        q[2] = p_i2;
-        q[3] = p_i3;
-    }
     if (tid < F) v.mbin[tid] = p_mb;
     for (int f = tid + nthr; f < F; f += nthr) v.mbin[f] = s.missing_bin[f];  // F > kPlanThreads
     if (tid < ne_old) v.eg[tid] = p_eg;  // the pairs' nodes: by the fold
@@ -5123,7 +5154,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
         if (tid < n_pairs) {
             v.wg[tid] = p_pg;
             v.wf[tid] = p_pf;
-            v.eg[pair_node(tid, p_bl)] = p_pf != 0x7FFFFFFF ? p_pg : -1.0;  // a found split has gain > 0
+            v.eg[pair_node(tid)] = p_pf != 0x7FFFFFFF ? p_pg : -1.0;  // a found split has gain > 0
         }
     } else {  // F <= 64
         // Bound by the instructions of 16 waves on one CU: a maximum of the
@@ -5143,7 +5174,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
             for (int k = K0; k < K1; ++k) {
                 const int pr = wvu + k * nwaves;
                 if (pr >= n_pairs) break;  // wave-uniform
-                const int e_id = pair_node(pr, bq[k]);
+                const int e_id = pair_node(pr);
                 const unsigned long long at =
                     __ballot((unsigned)((unsigned long long)__double_as_longlong(gq[k]) >> 32) == mh[k - K0]);
                 if (mh[k - K0] != 0u && (at & (at - 1ULL)) == 0ULL) {
@@ -5220,7 +5251,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
         }
         const int pr = tid - 64;
         if (pr < n_pairs) {
-            const int e_id = pair_node(pr, root_mode ? 0 : v.it[pr >> 1].builds_left);
+            const int e_id = pair_node(pr);
             const ScanResult *base = &s.scan[(size_t)pr * F];
             const int bf = v.wf[pr];
             const bool found = bf != 0x7FFFFFFF;
@@ -5314,6 +5345,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
             b.n_acc = 0;
             b.chunk_p = b.chunk_a = 0;
             b.slices = 1;
+            b.left[0] = b.left[1] = 0u;
             *s.batch = b;
             if (host != nullptr) publish_header(host, b);
         }
@@ -5681,7 +5713,8 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
         finish(4);
         return;
     }
-    for (int jj = tid; jj < nsel; jj += nthr) {
+    unsigned long long built_left = 0ULL;
+    for (int jj = tid; jj < nsel; jj += nthr) {  // lanes of wave 0 (nsel <= 64)
         const int Xs = v.sel_e[jj];
         ENode *e = &s.enodes[Xs];
         const SelNode &sn = v.sn[jj];
@@ -5689,6 +5722,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
         const int64_t m = e0 - b0;
         const int ebuf = sn.buf, ehist = sn.hist, edep = sn.depth;
         const bool bl = nlft <= m - nlft;
+        built_left = __ballot(bl);
         const int le = ne + 2 * jj, hb = g0.n_hist + jj;
         Item it;
         it.begin = b0;
@@ -5788,6 +5822,8 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
         b.chunk_p = (int32_t)chunk_p;
         b.chunk_a = (int32_t)chunk;
         b.slices = total * s.acc_slices * s.n_tiles <= s.slice_blocks && !s.rcp ? s.acc_slices : 1;
+        b.left[0] = (uint32_t)built_left;
+        b.left[1] = (uint32_t)(built_left >> 32);
         *s.batch = b;
         if (host != nullptr) publish_header(host, b);
     }

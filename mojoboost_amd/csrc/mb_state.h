@@ -86,6 +86,7 @@ struct Batch {
     int32_t chunk_p;   // parent rows per partition task
     int32_t chunk_a;   // accumulated rows per accumulation task
     int32_t slices;    // feature slices an accumulation task is split into (1: none)
+    uint32_t left[2];  // bit j: item j accumulates its left child (at most 64 items)
 };
 
 // Replay state of the best-first order (touched by the planning block only).
