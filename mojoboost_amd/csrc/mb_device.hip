@@ -28,6 +28,7 @@
 #include "mb_host.h"
 #include "mb_kernels.h"
 #include "mb_math.h"
+#include "mb_plan.h"
 #include "mb_state.h"
 
 namespace {
@@ -637,6 +638,10 @@ struct TrainBuffers {
     int T = 0, L = 0, max_nodes = 0;
 };
 
+[[noreturn]] void refuse_planner() {
+    throw Error{MOJOTREES_ERROR_UNSUPPORTED, "num_leaves * n_features too large for the planner's LDS (160 KiB)"};
+}
+
 TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t last_round = 0) {
     TrainBuffers tb;
     const int K = p->objective == MBH_OBJ_MULTICLASS ? p->num_class : 1;
@@ -919,9 +924,7 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
 
     // the fp32 path's binary32 derivatives, interleaved per row
     if (!quantized && !hp.grad64) s.gh2 = dalloc<float>(2 * (size_t)ds->n, run.arena);
-    if (mb::plan_lds_bytes(s) > 160 * 1024)
-        throw Error{MOJOTREES_ERROR_UNSUPPORTED,
-                    "num_leaves * n_features too large for the planner's LDS (160 KiB)"};
+    if (!mb::plan_fits(L, mb::plan_lds_bytes(s), 0)) refuse_planner();
     if (mb::hist_lds_bytes(s) + kPbStaticLds > 160 * 1024)
         throw Error{MOJOTREES_ERROR_TRAINING, "internal: the feature tile exceeds one workgroup's LDS"};
     HIPX(hipMemset(s.rows0, 0, (size_t)ds->n * sizeof(int32_t)));
@@ -1277,6 +1280,9 @@ int32_t mbh_train(mbh_dataset *ds, const mbh_params *p, mbh_fit **out, char *err
         Run run(ds);
         TrainBuffers tb = setup_state(ds, p, run);
         mb::DevState &s = tb.s;
+        bool fits = false;  // (calls that grow no tree do not launch the planner)
+        HIPX(mb::planner_fits(s, &fits));
+        if (!fits) refuse_planner();
         setup_record_partition(s, ds, p, run);
         const int K = s.hp.num_class;
         fit->num_class = K;

@@ -28,6 +28,8 @@ inline int acc_kind(const HyperParams &hp) { return hp.wide ? kAccWide : hp.quan
 // accumulation LDS of a tile of tile_f features
 size_t pb_lds_bytes_for(int tile_f, int lds_stride, int kind);
 size_t plan_lds_bytes(const DevState &s);
+// Whether the planner can grow s's trees (its dynamic and own LDS, its slots).
+hipError_t planner_fits(const DevState &s, bool *fits);
 size_t score_lds_bytes(const DevState &s);
 size_t rank_lds_bytes(const DevState &s);
 // With both events given, the runtime records them at the kernel's own start

@@ -34,6 +34,7 @@
 
 #include "mb_kernels.h"
 #include "mb_math.h"
+#include "mb_plan.h"
 #include "mb_state.h"
 
 namespace mb {
@@ -4691,55 +4692,6 @@ __global__ __launch_bounds__(kFoldThreads) void k_fold(DevState s, int root_mode
 //    replay will take, so speculative expansions are mostly used.
 constexpr int kPlanThreads = 1024;
 
-// LDS layout of the planner (byte offsets), shared by the host's size query
-// and the kernel.
-// The fields of a selected leaf's explored node the batch setup needs.
-struct SelNode {
-    int64_t begin, end, n_left;
-    int32_t buf, hist, depth, feature, bin, default_left, cat, pad_;
-};
-
-struct PlanLayout {
-    size_t sn, mbin;
-    size_t wg, eg, cb, kr, wf, el, ep, rw, fr, ci, sl_e, sl_fid, cm_e, cm_fid, cm_lf, sel_e, pcnt, poff, qcnt, qoff;
-    size_t total;
-};
-
-__host__ __device__ inline PlanLayout plan_layout(int L, int E, int K, int F) {
-    PlanLayout p;
-    size_t o = 0;
-    auto take = [&o](size_t bytes, size_t align) {
-        o = (o + align - 1) & ~(align - 1);
-        const size_t at = o;
-        o += bytes;
-        return at;
-    };
-    p.wg = take((size_t)8 * 2 * K, 8);       // pair's best gain
-    p.eg = take((size_t)8 * E, 8);           // explored node's gain view
-    p.cb = take((size_t)8 * E, 8);           // replay: explored node's bar; selection: bottleneck values
-    p.kr = take((size_t)8 * E, 8);           // replay: a step's right children; selection: fr, ci
-    p.fr = p.kr;                             // in the committed frontier
-    p.ci = p.kr + (size_t)4 * E;             // jump pointers, then candidates' node ids
-    p.wf = take((size_t)4 * 2 * K, 4);       // pair's best feature
-    p.el = take((size_t)4 * E, 4);           // explored node's left child
-    p.ep = take((size_t)4 * E, 4);           // explored node's parent
-    p.rw = take((size_t)4 * E, 4);           // explored node's rows
-    p.sl_e = take((size_t)4 * L, 4);
-    p.sl_fid = take((size_t)4 * L, 4);
-    p.cm_e = take((size_t)4 * L, 4);
-    p.cm_fid = take((size_t)4 * L, 4);
-    p.cm_lf = take((size_t)4 * L, 4);
-    p.sel_e = take((size_t)4 * K, 4);
-    p.pcnt = take((size_t)4 * K, 4);
-    p.poff = take((size_t)4 * (K + 1), 4);
-    p.qcnt = take((size_t)4 * K, 4);
-    p.qoff = take((size_t)4 * (K + 1), 4);
-    p.sn = take(sizeof(SelNode) * K, 16);    // the selected leaves' nodes
-    p.mbin = take((size_t)4 * F, 4);         // missing bin per feature
-    p.total = o;
-    return p;
-}
-
 struct PlanView {
     SelNode *sn;
     int32_t *mbin;
@@ -5213,7 +5165,7 @@ __global__ __launch_bounds__(kPlanThreads) void k_plan(DevState s, int root_mode
         int nl = nl0, nn = g0.n_nodes, nc = 0, done = 0, x = -1;
         if (L <= 64) replay_wave<1>(v, L, nl, nn, nc, done, x);
         else if (L <= 256) replay_wave<4>(v, L, nl, nn, nc, done, x);
-        else replay_wave<8>(v, L, nl, nn, nc, done, x);  // L <= 512: the LDS of more nodes is not there
+        else replay_wave<kPlanSlots / 64>(v, L, nl, nn, nc, done, x);
         if (lane == 0) {
             s_nc = nc;
             s_done = done;
@@ -6378,6 +6330,12 @@ size_t pb_lds_bytes_for(int tile_f, int lds_stride, int kind) {
 size_t hist_lds_bytes(const DevState &s) { return pb_lds_bytes_for(s.tile_f, s.lds_stride, acc_kind(s.hp)); }
 size_t plan_lds_bytes(const DevState &s) {
     return plan_layout(s.hp.num_leaves, s.e_cap, s.kmax, s.n_features).total;
+}
+hipError_t planner_fits(const DevState &s, bool *fits) {
+    hipFuncAttributes a{};
+    const hipError_t e = hipFuncGetAttributes(&a, (const void *)k_plan);
+    if (e == hipSuccess) *fits = plan_fits(s.hp.num_leaves, plan_lds_bytes(s), a.sharedSizeBytes);
+    return e;
 }
 
 #define MB_SET_LDS(fn, bytes)                                                                     \
