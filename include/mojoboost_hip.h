@@ -162,7 +162,10 @@ int32_t mbh_bin_dense_device(const double *data, int64_t n_rows, int32_t n_featu
 int32_t mbh_device_count(void);
 
 /* Upload a binned matrix and its labels; builds the per-row records
- * (F bin bytes + 2 gradient bytes, padded to a power of two). */
+ * (F bin bytes + 2 gradient bytes, padded to a power of two). A call on a
+ * dataset leaves its working memory on the device to the dataset's next call
+ * (at most 4 GiB over all datasets), until mbh_dataset_free or until an
+ * allocation of this library needs it. */
 int32_t mbh_dataset_create(const uint8_t *bins_cm, int64_t n_rows,
                            int32_t n_features, int32_t n_bins,
                            const int32_t *missing_bin, const double *labels,

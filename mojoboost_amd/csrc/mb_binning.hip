@@ -31,6 +31,7 @@
 #include "../../include/mojoboost_hip.h"
 #include "../../include/mojotrees.h"
 #include "mb_host.h"
+#include "mb_memory.h"
 
 namespace {
 
@@ -126,7 +127,7 @@ struct Buffers {
     template <class T>
     T *alloc(size_t count) {
         void *q = nullptr;
-        HIPB(hipMalloc(&q, count * sizeof(T) > 0 ? count * sizeof(T) : 1));
+        HIPB(mb::device_malloc(&q, count * sizeof(T) > 0 ? count * sizeof(T) : 1));
         p.push_back(q);
         return (T *)q;
     }

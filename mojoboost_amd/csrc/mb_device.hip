@@ -18,8 +18,6 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
-#include <memory>
-#include <mutex>
 #include <string>
 #include <vector>
 
@@ -28,6 +26,7 @@
 #include "mb_host.h"
 #include "mb_kernels.h"
 #include "mb_math.h"
+#include "mb_memory.h"
 #include "mb_plan.h"
 #include "mb_state.h"
 
@@ -55,124 +54,16 @@ T *dalloc(size_t count, std::vector<void *> &owned) {
     void *p = nullptr;
     size_t bytes = count * sizeof(T);
     if (bytes == 0) bytes = sizeof(T);
-    HIPX(hipMalloc(&p, bytes));
+    HIPX(mb::device_malloc(&p, bytes));
     owned.push_back(p);
     return (T *)p;
 }
 
-// Device memory of the library's calls on a dataset. A call places its
-// buffers in slabs (Arena) instead of allocating each one, and leaves the
-// slabs to the dataset's next call: a training places some 100 buffers, and
-// allocating and freeing them took 0.5 ms on a small table and 6 ms for ten
-// classes on 300K x 50. Idle slabs belong to their dataset, are freed with
-// it, total at most kIdleMost over the process, and are all freed when an
-// allocation fails. Calls on one dataset at a time share nothing: a call takes
-// every idle slab of its dataset, a second one beside it finds none.
-struct Slab {
-    uint8_t *p = nullptr;
-    size_t size = 0;
-    const void *owner = nullptr;
-};
-
-class SlabPool {
-public:
-    std::vector<Slab> take(const void *owner) {
-        std::lock_guard<std::mutex> lock(mu_);
-        std::vector<Slab> mine;
-        for (size_t i = idle_.size(); i-- > 0;)
-            if (idle_[i].owner == owner) {
-                mine.insert(mine.begin(), idle_[i]);
-                bytes_ -= idle_[i].size;
-                idle_.erase(idle_.begin() + (ptrdiff_t)i);
-            }
-        return mine;
-    }
-    // the slabs must be idle on the device
-    void give(std::vector<Slab> &slabs) {
-        std::lock_guard<std::mutex> lock(mu_);
-        for (const Slab &s : slabs) {
-            if (s.owner && bytes_ + s.size <= kIdleMost) {
-                idle_.push_back(s);
-                bytes_ += s.size;
-            } else {
-                (void)hipFree(s.p);
-            }
-        }
-        slabs.clear();
-    }
-    // an owner's idle slabs, or every one
-    void drop(const void *owner, bool all = false) {
-        std::lock_guard<std::mutex> lock(mu_);
-        for (size_t i = idle_.size(); i-- > 0;)
-            if (all || idle_[i].owner == owner) {
-                (void)hipFree(idle_[i].p);
-                bytes_ -= idle_[i].size;
-                idle_.erase(idle_.begin() + (ptrdiff_t)i);
-            }
-    }
-
-private:
-    static constexpr size_t kIdleMost = (size_t)4 << 30;
-    std::mutex mu_;
-    std::vector<Slab> idle_;
-    size_t bytes_ = 0;
-};
-
-// Never destroyed: the HIP runtime may be gone when static objects are.
-SlabPool &slab_pool() {
-    static SlabPool *pool = new SlabPool();
-    return *pool;
-}
-
-// The buffers of one call, in the slabs its dataset's last call left and in
-// new ones.
-class Arena {
-public:
-    explicit Arena(const void *owner) : owner_(owner) {
-        if (owner) slabs_ = slab_pool().take(owner);
-    }
-    Arena(const Arena &) = delete;
-    Arena &operator=(const Arena &) = delete;
-    ~Arena() {
-        // as the frees did, wait for whatever still uses the buffers
-        if (!slabs_.empty()) (void)hipDeviceSynchronize();
-        slab_pool().give(slabs_);
-    }
-    void *place(size_t bytes) {
-        bytes = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
-        // first fit over the slabs' free ends
-        used_.resize(slabs_.size(), 0);
-        for (size_t i = 0; i < slabs_.size(); ++i)
-            if (slabs_[i].size - used_[i] >= bytes) {
-                void *at = slabs_[i].p + used_[i];
-                used_[i] += bytes;
-                return at;
-            }
-        Slab s;
-        s.owner = owner_;
-        s.size = std::max(bytes, kSlab);
-        hipError_t e = hipMalloc((void **)&s.p, s.size);
-        if (e != hipSuccess) {
-            (void)hipGetLastError();
-            slab_pool().drop(nullptr, true);
-            s.size = bytes;
-            HIPX(hipMalloc((void **)&s.p, s.size));
-        }
-        slabs_.push_back(s);
-        used_.push_back(bytes);
-        return s.p;
-    }
-
-private:
-    static constexpr size_t kSlab = (size_t)32 << 20;
-    const void *owner_;
-    std::vector<Slab> slabs_;
-    std::vector<size_t> used_;
-};
-
 template <class T>
-T *dalloc(size_t count, Arena &arena) {
-    return (T *)arena.place(count * sizeof(T));
+T *dalloc(size_t count, mb::Arena &arena) {
+    void *p = nullptr;
+    HIPX(arena.place(count * sizeof(T), &p));
+    return (T *)p;
 }
 
 int device_count_gfx950() {
@@ -252,7 +143,7 @@ struct mbh_dataset {
     int max_query = 0;
     std::vector<void *> owned;
     ~mbh_dataset() {
-        slab_pool().drop(this);
+        mb::slab_pool().drop(this);
         for (void *p : owned) (void)hipFree(p);
     }
 };
@@ -315,7 +206,7 @@ struct mbh_fit {
 namespace {
 
 struct Run {
-    Arena arena;
+    mb::Arena arena;
     explicit Run(const mbh_dataset *ds) : arena(ds) {}
 };
 

@@ -37,6 +37,7 @@
 
 #include "../../include/mojoboost_hip.h"
 #include "../../include/mojotrees.h"
+#include "mb_memory.h"
 #include "mb_trees.h"
 
 namespace {
@@ -359,7 +360,7 @@ extern "C" int32_t mbh_predict_binned(const uint8_t *bins_cm, int64_t n, int32_t
         auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
         const size_t at_bins = up(im.bytes.size()), at_out = at_bins + up((size_t)F * m0);
         DeviceBlock d;
-        HIPP(hipMalloc((void **)&d.p, at_out + (size_t)m0 * K * sizeof(double)));
+        HIPP(mb::device_malloc((void **)&d.p, at_out + (size_t)m0 * K * sizeof(double)));
         if (!im.bytes.empty()) HIPP(hipMemcpyAsync(d.p, im.bytes.data(), im.bytes.size(), hipMemcpyHostToDevice, 0));
         a.bins = d.p + at_bins;
         a.out = (double *)(d.p + at_out);
