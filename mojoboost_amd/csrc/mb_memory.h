@@ -8,6 +8,7 @@
 #include <cstddef>
 #include <cstdint>
 #include <mutex>
+#include <new>
 #include <vector>
 
 namespace mb {
@@ -29,22 +30,39 @@ struct Slab {
 
 class SlabPool {
 public:
-    std::vector<Slab> take(const void *owner) {
+    // no exception leaves these two: without host memory for the list, a call
+    // starts with no slab, and a slab is freed instead of kept
+    std::vector<Slab> take(const void *owner) noexcept {
         std::lock_guard<std::mutex> lock(mu_);
         std::vector<Slab> mine;
-        for (size_t i = idle_.size(); i-- > 0;)
-            if (idle_[i].owner == owner) {
-                mine.insert(mine.begin(), idle_[i]);
-                bytes_ -= idle_[i].size;
-                idle_.erase(idle_.begin() + (ptrdiff_t)i);
+        try {
+            mine.reserve(idle_.size());
+        } catch (const std::bad_alloc &) {
+            return mine;
+        }
+        size_t kept = 0;
+        for (const Slab &s : idle_) {
+            if (s.owner == owner) {
+                mine.push_back(s);
+                bytes_ -= s.size;
+            } else {
+                idle_[kept++] = s;
             }
+        }
+        idle_.resize(kept);
         return mine;
     }
     // the slabs must be idle on the device
-    void give(std::vector<Slab> &slabs) {
+    void give(std::vector<Slab> &slabs) noexcept {
         std::lock_guard<std::mutex> lock(mu_);
+        bool room = true;
+        try {
+            idle_.reserve(idle_.size() + slabs.size());
+        } catch (const std::bad_alloc &) {
+            room = false;
+        }
         for (const Slab &s : slabs) {
-            if (s.owner && bytes_ + s.size <= kIdleMost) {
+            if (room && s.owner && bytes_ + s.size <= kIdleMost) {
                 idle_.push_back(s);
                 bytes_ += s.size;
             } else {
@@ -107,8 +125,14 @@ public:
         if (!slabs_.empty()) (void)hipDeviceSynchronize();
         slab_pool().give(slabs_);
     }
-    hipError_t place(size_t bytes, void **at) {
+    hipError_t place(size_t bytes, void **at) noexcept {
         bytes = (std::max<size_t>(bytes, 1) + 255) & ~(size_t)255;
+        try {
+            slabs_.reserve(slabs_.size() + 1);
+            used_.reserve(slabs_.size() + 1);
+        } catch (const std::bad_alloc &) {
+            return hipErrorOutOfMemory;
+        }
         // first fit over the slabs' free ends
         used_.resize(slabs_.size(), 0);
         for (size_t i = 0; i < slabs_.size(); ++i)

@@ -1,7 +1,8 @@
 """Device allocation and the slabs (mb_memory.h) against a small fake card,
 compiled for the host: an allocation that does not fit beside the idle slabs
 frees them and succeeds, a call whose dataset left slabs of other sizes frees
-its own unused ones, memory in use stays, and what cannot fit fails cleanly."""
+its own unused ones, memory in use stays, what cannot fit fails cleanly, and
+no exception leaves them where the host has no memory."""
 import subprocess
 from pathlib import Path
 
@@ -108,6 +109,49 @@ int main() {
 """
 
 
+NO_HOST_MEMORY = r"""
+#include <cstdio>
+#include <cstdlib>
+#include <new>
+static bool no_memory = false;
+void *operator new(std::size_t n) {
+    if (no_memory) throw std::bad_alloc();
+    return std::malloc(n ? n : 1);
+}
+void operator delete(void *p) noexcept { std::free(p); }
+void operator delete(void *p, std::size_t) noexcept { std::free(p); }
+#include "mb_memory.h"
+using namespace mb;
+#define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); std::exit(1); } } while (0)
+int main() {
+    card.total = (size_t)1 << 30;
+    int owner = 0;
+    void *p = nullptr;
+    {
+        Arena run(&owner);
+        CHECK(run.place(100, &p) == hipSuccess);
+        no_memory = true;  // while the call ends
+    }
+    CHECK(card.used == 0);
+    {
+        Arena run(&owner);
+        CHECK(run.place(100, &p) == hipErrorOutOfMemory && card.used == 0);
+        no_memory = false;
+        CHECK(run.place(100, &p) == hipSuccess);
+    }
+    CHECK(card.used == (size_t)32 << 20);
+    no_memory = true;  // while the call begins: the slab stays idle
+    {
+        Arena run(&owner);
+        no_memory = false;
+        CHECK(run.place(100, &p) == hipSuccess && card.used == (size_t)64 << 20);
+    }
+    CHECK(slab_pool().drop(&owner) == (size_t)64 << 20 && card.used == 0);
+    return 0;
+}
+"""
+
+
 @pytest.fixture(scope="module")
 def build(tmp_path_factory):
     at = tmp_path_factory.mktemp("memory")
@@ -125,6 +169,11 @@ def build(tmp_path_factory):
 
 def test_allocation_frees_idle_slabs(build):
     out = build(PROGRAM)
+    assert out.returncode == 0, out.stdout + out.stderr
+
+
+def test_no_exception_without_host_memory(build):
+    out = build(NO_HOST_MEMORY)
     assert out.returncode == 0, out.stdout + out.stderr
 
 
