@@ -150,42 +150,6 @@ struct mbh_dataset {
 
 constexpr int kNumStats = 22;
 
-// A fit's raw scores on the host: pinned from kPinBytes on (the copy from the
-// device then runs at the link's rate, 84 MB in 1.6 ms against 5 into
-// pageable memory after 14 of zeroing a vector), else ordinary memory,
-// not zeroed first.
-struct HostScores {
-    double *p = nullptr;
-    size_t n = 0;
-    bool pinned = false;
-    void reserve(size_t count) {
-        release();
-        if (count * sizeof(double) >= kPinBytes) {
-            pinned = hipHostMalloc((void **)&p, count * sizeof(double), hipHostMallocDefault) == hipSuccess;
-            if (!pinned) {
-                (void)hipGetLastError();
-                p = nullptr;
-            }
-        }
-        if (!p) p = new double[count > 0 ? count : 1];
-        n = count;
-    }
-    void release() {
-        if (pinned) (void)hipHostFree(p);
-        else delete[] p;
-        p = nullptr;
-        n = 0;
-        pinned = false;
-    }
-    HostScores() = default;
-    HostScores(const HostScores &) = delete;
-    HostScores &operator=(const HostScores &) = delete;
-    ~HostScores() { release(); }
-
-private:
-    static constexpr size_t kPinBytes = (size_t)1 << 20;
-};
-
 struct mbh_fit {
     int num_class = 1;
     int objective = 0;
@@ -196,7 +160,7 @@ struct mbh_fit {
     std::vector<int32_t> feature, threshold, left, right, default_left, missing_bin;
     std::vector<double> value, gain, count;
     std::vector<uint64_t> cat_bits;  // 4 words per node
-    HostScores train_raw;
+    mb::HostScores train_raw;
     double stats[kNumStats] = {0};
     // time_histograms runs: per expansion launch, (tree, iteration, rows
     // partitioned, rows accumulated, partition ms, accumulation ms)

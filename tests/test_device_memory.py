@@ -2,7 +2,8 @@
 compiled for the host: an allocation that does not fit beside the idle slabs
 frees them and succeeds, a call whose dataset left slabs of other sizes frees
 its own unused ones, memory in use stays, what cannot fit fails cleanly, and
-no exception leaves them where the host has no memory."""
+no exception leaves them where the host has no memory. The scores of the fits
+alive together pin a bounded part of the host's memory."""
 import subprocess
 from pathlib import Path
 
@@ -35,6 +36,22 @@ inline hipError_t hipFree(void *p) {
     if (!card.live.count(p)) std::abort();
     card.used -= card.live[p];
     card.live.erase(p);
+    return hipSuccess;
+}
+enum { hipHostMallocDefault };
+inline size_t pinned = 0, refuse_pinned = 0;
+inline std::map<void *, size_t> pinned_live;
+inline hipError_t hipHostMalloc(void **p, size_t n, unsigned) {
+    if (refuse_pinned) return card.last = hipErrorOutOfMemory;
+    pinned += n;
+    pinned_live[*p = std::malloc(n)] = n;
+    return hipSuccess;
+}
+inline hipError_t hipHostFree(void *p) {
+    if (!pinned_live.count(p)) std::abort();
+    pinned -= pinned_live[p];
+    pinned_live.erase(p);
+    std::free(p);
     return hipSuccess;
 }
 inline hipError_t hipDeviceSynchronize() { return ++card.syncs, hipSuccess; }
@@ -152,6 +169,47 @@ int main() {
 """
 
 
+PINNED = r"""
+#include <cstdio>
+#include <memory>
+#include "mb_memory.h"
+using namespace mb;
+#define CHECK(x) do { if (!(x)) { std::printf("line %d: %s\n", __LINE__, #x); std::exit(1); } } while (0)
+int main() {
+    const size_t count = (size_t)12 << 20;  // 96 MB a fit
+    {
+        std::vector<std::unique_ptr<HostScores>> fits;
+        for (int i = 0; i < 30; ++i) {
+            fits.emplace_back(new HostScores());
+            fits.back()->reserve(count);
+            fits.back()->p[count - 1] = i;
+            CHECK(pinned <= (size_t)1 << 30 && fits.back()->n == count);
+        }
+        CHECK(pinned == 10 * 8 * count);  // the first ten
+        fits.erase(fits.begin(), fits.begin() + 3);
+        CHECK(pinned == 7 * 8 * count);
+        fits.emplace_back(new HostScores());
+        fits.back()->reserve(count);
+        CHECK(pinned == 8 * 8 * count);  // room again
+        fits.back()->reserve(100);
+        CHECK(pinned == 7 * 8 * count && fits.back()->n == 100);  // small ones are not pinned
+        fits.back()->reserve(0);
+        refuse_pinned = 1;
+        fits.back()->reserve(count);
+        CHECK(pinned == 7 * 8 * count && fits.back()->p && card.last == hipSuccess);
+        refuse_pinned = 0;
+    }
+    CHECK(pinned == 0);
+    HostScores a, b;
+    a.reserve(((size_t)1 << 30) / 8);  // all of it
+    CHECK(pinned == (size_t)1 << 30);
+    b.reserve((size_t)1 << 18);
+    CHECK(pinned == (size_t)1 << 30);
+    return 0;
+}
+"""
+
+
 @pytest.fixture(scope="module")
 def build(tmp_path_factory):
     at = tmp_path_factory.mktemp("memory")
@@ -174,6 +232,11 @@ def test_allocation_frees_idle_slabs(build):
 
 def test_no_exception_without_host_memory(build):
     out = build(NO_HOST_MEMORY)
+    assert out.returncode == 0, out.stdout + out.stderr
+
+
+def test_fits_alive_pin_a_bounded_total(build):
+    out = build(PINNED)
     assert out.returncode == 0, out.stdout + out.stderr
 
 
