@@ -32,6 +32,7 @@
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
+#include "mb_grid.h"
 #include "mb_kernels.h"
 #include "mb_math.h"
 #include "mb_plan.h"
@@ -403,7 +404,7 @@ __global__ __launch_bounds__(kRankThreads) void k_lambdarank(DevState s) {
     const uint64_t bstream = hp.bagging ? bag_stream_of(hp, rd.round) : 0;
     const int64_t bfall = hp.bagging ? bag_fallback_of(s, rd.round) : -1;
     double mg = 0.0, mh = 0.0;
-    for (int qi = blockIdx.x; qi < s.n_small; qi += gridDim.x) {
+    for (unsigned qi = blockIdx.x; qi < (unsigned)s.n_small; qi += gridDim.x) {
         const int q = s.rank_order[qi];
         const int64_t a = s.qstart[q];
         const int cnt = (int)(s.qstart[q + 1] - a);
@@ -6255,8 +6256,8 @@ hipError_t launch_objective(const DevState &s, int grid, hipStream_t st) {
     if (s.hp.objective == kObjLambdarank) {
         // a block per query, as many as may be in flight; the next queries
         // of rank_order go to the blocks that end first
-        const int g = s.n_small > 1 ? s.n_small : 1;
-        hipLaunchKernelGGL(k_lambdarank, dim3(g), dim3(kRankThreads), rank_lds_bytes(s), st, s);
+        hipLaunchKernelGGL(k_lambdarank, dim3(launch_blocks(s.n_small, kRankThreads)), dim3(kRankThreads),
+                           rank_lds_bytes(s), st, s);
         if (s.n_big > 0) {
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
