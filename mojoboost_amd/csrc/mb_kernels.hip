@@ -6220,18 +6220,22 @@ __global__ __launch_bounds__(256) void k_build_records(const uint8_t *bins_cm, u
 // of a block through LDS, a run of classes at a time, so both sides move
 // consecutive values.
 constexpr int kRowMajorK = 16;
+constexpr int kRowMajorBlocks = 1 << 16;
+static_assert((int64_t)kRowMajorBlocks * 256 < (int64_t)1 << 32, "a dimension's threads");
 __global__ __launch_bounds__(256) void k_row_major(const double *__restrict__ in, double *__restrict__ out, int64_t n,
                                                    int K) {
     __shared__ double t[64][kRowMajorK + 1];
-    const int64_t r0 = (int64_t)blockIdx.x * 64;
-    const int rows = (int)(n - r0 < 64 ? n - r0 : 64);
     const int k0 = (int)blockIdx.y * kRowMajorK, ks = min(kRowMajorK, K - k0);
-    for (int i = threadIdx.x; i < 64 * ks; i += 256)
-        if ((i & 63) < rows) t[i & 63][i >> 6] = in[(size_t)(k0 + (i >> 6)) * n + r0 + (i & 63)];
-    __syncthreads();
-    for (int i = threadIdx.x; i < rows * ks; i += 256) {
-        const int r = i / ks, k = i - r * ks;
-        out[(size_t)(r0 + r) * K + k0 + k] = t[r][k];
+    for (int64_t r0 = (int64_t)blockIdx.x * 64; r0 < n; r0 += (int64_t)gridDim.x * 64) {
+        const int rows = (int)(n - r0 < 64 ? n - r0 : 64);
+        for (int i = threadIdx.x; i < 64 * ks; i += 256)
+            if ((i & 63) < rows) t[i & 63][i >> 6] = in[(size_t)(k0 + (i >> 6)) * n + r0 + (i & 63)];
+        __syncthreads();
+        for (int i = threadIdx.x; i < rows * ks; i += 256) {
+            const int r = i / ks, k = i - r * ks;
+            out[(size_t)(r0 + r) * K + k0 + k] = t[r][k];
+        }
+        __syncthreads();  // the tile is the next rows'
     }
 }
 
@@ -6562,8 +6566,9 @@ hipError_t launch_build_records(const uint8_t *bins_cm, uint8_t *records, int64_
     return hipGetLastError();
 }
 hipError_t launch_row_major(const double *in, double *out, int64_t n, int K, hipStream_t st) {
-    hipLaunchKernelGGL(k_row_major, dim3((unsigned)((n + 63) / 64), (unsigned)((K + kRowMajorK - 1) / kRowMajorK)),
-                       dim3(256), 0, st, in, out, n, K);
+    const unsigned grid = (unsigned)std::min<int64_t>((n + 63) / 64, kRowMajorBlocks);
+    hipLaunchKernelGGL(k_row_major, dim3(grid, (unsigned)((K + kRowMajorK - 1) / kRowMajorK)), dim3(256), 0, st, in,
+                       out, n, K);
     return hipGetLastError();
 }
 hipError_t launch_fill_f64(double *p, int64_t n, int K, const double *base, int grid, hipStream_t st) {
