@@ -31,6 +31,7 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -253,15 +254,29 @@ struct DeviceBlock {
     }
 };
 
+size_t up(size_t b) { return (b + 255) & ~(size_t)255; }
+
 // The host's image of everything but the bins and the scores, uploaded as
-// one copy; parts are placed at 256-byte offsets.
+// one copy; parts are placed at 256-byte offsets and written in place (memory
+// of a call's own: zeroing it and copying the parts together cost a few
+// milliseconds per million nodes).
 struct Image {
-    std::vector<uint8_t> bytes;
+    std::unique_ptr<uint8_t[]> bytes;
+    size_t size = 0, room = 0;
+    // at most `total` bytes in `parts` parts
+    Image(size_t total, int parts) : bytes(new uint8_t[total + (size_t)parts * 256]), room(total + (size_t)parts * 256) {}
+    template <class T>
+    T *part(size_t count, size_t &at) {
+        at = up(size);
+        size = at + count * sizeof(T);
+        if (size > room) throw Error{MOJOTREES_ERROR_TRAINING, "internal: prediction image"};
+        return (T *)(bytes.get() + at);
+    }
     template <class T>
     size_t put(const T *src, size_t count) {
-        const size_t at = (bytes.size() + 255) & ~(size_t)255;
-        bytes.resize(at + std::max<size_t>(count, 1) * sizeof(T));
-        if (count) std::memcpy(bytes.data() + at, src, count * sizeof(T));
+        size_t at;
+        T *to = part<T>(count, at);
+        if (count) std::memcpy(to, src, count * sizeof(T));
         return at;
     }
 };
@@ -325,43 +340,46 @@ extern "C" int32_t mbh_predict_binned(const uint8_t *bins_cm, int64_t n, int32_t
         a.K = K;
         a.learning_rate = learning_rate;
         a.log_rows = lg;
-        Image im;
-        Packed p;
-        auto place = [&](int32_t f) { return lds_bins ? (uint32_t)(((f >> 2) << (lg + 2)) + (f & 3)) : (uint32_t)f; };
-        const bool packed = F <= 65536 && pack_trees(e, shapes, K, rows ? kTreeCap : std::min(kTreeCap, kLeafCap >> lg), place, p);
+        const int64_t T = tree_end - tree_begin, o0 = node_offset[tree_begin], nn = node_offset[tree_end] - o0;
+        const size_t cat_words = cat_bits ? (size_t)nn * 4 : 0;
         size_t o_base = 0, o_cat = 0, o_words = 0, o_tree = 0, o_chunk = 0, o_of = 0, o_nodes = 0, o_md = 0,
                o_value = 0, o_root = 0;
-        if (base) o_base = im.put(base, K);
+        auto place = [&](int32_t f) { return lds_bins ? (uint32_t)(((f >> 2) << (lg + 2)) + (f & 3)) : (uint32_t)f; };
+        std::unique_ptr<Image> im;
+        Packed p;
+        bool packed = false;
+        if (F <= 65536 && chunks_hold(shapes)) {
+            im.reset(new Image((size_t)shapes.words * 8 + cat_words * 8 + (size_t)T * (4 + sizeof(Chunk)) +
+                                   (size_t)K * 12 + 4, 6));
+            unsigned long long *words = im->part<unsigned long long>((size_t)shapes.words, o_words);
+            unsigned long long *cat = cat_bits ? im->part<unsigned long long>(cat_words, o_cat) : nullptr;
+            packed = pack_trees(e, shapes, K, rows ? kTreeCap : std::min(kTreeCap, kLeafCap >> lg), place, words, cat, p);
+        }
         if (packed) {
-            o_words = im.put(p.words.data(), p.words.size());
-            o_tree = im.put(p.tree.data(), p.tree.size());
-            o_chunk = im.put(p.chunk.data(), p.chunk.size());
-            o_of = im.put(p.chunk_of.data(), p.chunk_of.size());
-            if (cat_bits) o_cat = im.put(p.cat.data(), p.cat.size());
+            o_tree = im->put(p.tree.data(), p.tree.size());
+            o_chunk = im->put(p.chunk.data(), p.chunk.size());
+            o_of = im->put(p.chunk_of.data(), p.chunk_of.size());
         } else {
-            const int64_t o0 = node_offset[tree_begin], nn = node_offset[tree_end] - o0;
-            std::vector<int4> nodes((size_t)nn);
-            std::vector<int32_t> md((size_t)nn), root((size_t)(tree_end - tree_begin));
+            im.reset(new Image((size_t)nn * (sizeof(int4) + 4 + 8) + cat_words * 8 + (size_t)T * 4 + (size_t)K * 8, 6));
+            int4 *nodes = im->part<int4>((size_t)nn, o_nodes);
+            int32_t *md = im->part<int32_t>((size_t)nn, o_md), *root = im->part<int32_t>((size_t)T, o_root);
             for (int64_t t = tree_begin; t < tree_end; ++t) {
                 const int64_t first = node_offset[t] - o0;
-                root[(size_t)(t - tree_begin)] = (int32_t)first;
+                root[t - tree_begin] = (int32_t)first;
                 for (int64_t i = node_offset[t]; i < node_offset[t + 1]; ++i) {
-                    nodes[(size_t)(i - o0)] = make_int4(feature[i] >= 0 ? feature[i] : -1, threshold[i],
-                                                        (int32_t)(first + left[i]), (int32_t)(first + right[i]));
-                    md[(size_t)(i - o0)] = missing_bin[i] * 2 + (default_left[i] ? 1 : 0);
+                    nodes[i - o0] = make_int4(feature[i] >= 0 ? feature[i] : -1, threshold[i],
+                                              (int32_t)(first + left[i]), (int32_t)(first + right[i]));
+                    md[i - o0] = missing_bin[i] * 2 + (default_left[i] ? 1 : 0);
                 }
             }
-            o_nodes = im.put(nodes.data(), nodes.size());
-            o_md = im.put(md.data(), md.size());
-            o_value = im.put(value + o0, (size_t)nn);
-            o_root = im.put(root.data(), root.size());
-            if (cat_bits) o_cat = im.put(cat_bits + (size_t)o0 * 4, (size_t)nn * 4);
+            o_value = im->put(value + o0, (size_t)nn);
+            if (cat_bits) o_cat = im->put(cat_bits + (size_t)o0 * 4, cat_words);
         }
-        auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-        const size_t at_bins = up(im.bytes.size()), at_out = at_bins + up((size_t)F * m0);
+        if (base) o_base = im->put(base, (size_t)K);
+        const size_t at_bins = up(im->size), at_out = at_bins + up((size_t)F * m0);
         DeviceBlock d;
         HIPP(mb::device_malloc((void **)&d.p, at_out + (size_t)m0 * K * sizeof(double)));
-        if (!im.bytes.empty()) HIPP(hipMemcpyAsync(d.p, im.bytes.data(), im.bytes.size(), hipMemcpyHostToDevice, 0));
+        if (im->size) HIPP(hipMemcpyAsync(d.p, im->bytes.get(), im->size, hipMemcpyHostToDevice, 0));
         a.bins = d.p + at_bins;
         a.out = (double *)(d.p + at_out);
         a.base = base ? (const double *)(d.p + o_base) : nullptr;
@@ -374,7 +392,7 @@ extern "C" int32_t mbh_predict_binned(const uint8_t *bins_cm, int64_t n, int32_t
         a.md = (const int32_t *)(d.p + o_md);
         a.value = (const double *)(d.p + o_value);
         a.root = (const int32_t *)(d.p + o_root);
-        a.n_trees = tree_end - tree_begin;
+        a.n_trees = T;
         a.max_steps = shapes.largest;
         const size_t lds = (size_t)kChunkWords * 8 + (rows ? 0 : (size_t)kLeafCap * 8) + (lds_bins ? row_bytes << lg : 0);
         const Kernel kernel = pick_kernel(rows, lds_bins, p.missing, cat_bits != nullptr);

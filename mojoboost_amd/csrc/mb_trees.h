@@ -48,11 +48,13 @@ struct Trees {
     const uint64_t *cat_bits;
 };
 
-// What one pass over the trees finds: the nodes of the largest one, and of
-// each its leaves and whether every right child follows its left one (the
-// trainer's order, which the chunks keep).
+// What one pass over the trees finds: the nodes of the largest one, the words
+// of the largest and of all (a word a node and one a leaf), and of each its
+// leaves and whether every right child follows its left one (the trainer's
+// order, which the chunks keep).
 struct Shapes {
     int32_t largest = 1;
+    int64_t most_words = 0, words = 0;
     std::vector<int32_t> leaves;
     std::vector<uint8_t> paired;
 };
@@ -86,32 +88,33 @@ inline Shapes check_trees(const Trees &e, int32_t F) {
         }
         s.leaves[(size_t)(t - e.t0)] = leaves;
         s.paired[(size_t)(t - e.t0)] = paired;
+        s.most_words = std::max(s.most_words, b - a + leaves);
+        s.words += b - a + leaves;
     }
     return s;
 }
 
-// The ensemble in chunks.
+// Whether every tree fits a chunk (and a word's place its 32 bits).
+inline bool chunks_hold(const Shapes &s) { return s.most_words <= kChunkWords && s.words < ((int64_t)1 << 31); }
+
+// The ensemble in chunks, beside their words.
 struct Packed {
-    std::vector<unsigned long long> words, cat;
     std::vector<uint32_t> tree;
     std::vector<Chunk> chunk;
     std::vector<int32_t> chunk_of;
     bool missing = false;
 };
 
-// Packs the trees, `place` giving a feature's place. False when one does not
-// fit: more words than a chunk's, or, siblings not next to each other, a node
-// reached twice, for which such a tree's words have no second place.
+// Packs trees that chunks_hold into sh.words words and, with category sets,
+// four words a node of `cat`; `place` gives a feature's place. False for a
+// tree that reaches a node twice, siblings not next to each other: its words
+// have no second place.
 template <class Place>
-bool pack_trees(const Trees &e, const Shapes &sh, int K, int max_chunk_trees, Place place, Packed &p) {
+bool pack_trees(const Trees &e, const Shapes &sh, int K, int max_chunk_trees, Place place, unsigned long long *packed,
+                unsigned long long *cat, Packed &p) {
     std::vector<int32_t> order, index;  // a tree's nodes, siblings next to each other
     std::vector<uint8_t> seen;
-    const int64_t nn = e.off[e.t1] - e.off[e.t0], T = e.t1 - e.t0;
-    int64_t n_words = nn;
-    for (const int32_t v : sh.leaves) n_words += v;
-    p.words.resize((size_t)n_words);
-    if (e.cat_bits) p.cat.resize((size_t)nn * 4);
-    p.tree.reserve((size_t)T);
+    p.tree.reserve((size_t)(e.t1 - e.t0));
     p.chunk_of.push_back(0);
     int32_t word0 = 0, node0 = 0;
     for (int k = 0; k < K; ++k) {
@@ -124,9 +127,8 @@ bool pack_trees(const Trees &e, const Shapes &sh, int K, int max_chunk_trees, Pl
                 nodes += c;
                 words += w;
             }
-            if (trees == 0) return false;
             p.chunk.push_back(Chunk{(int32_t)p.tree.size(), trees, word0, words, node0, 0});
-            unsigned long long *nw = p.words.data() + word0, *values = nw + nodes;
+            unsigned long long *nw = packed + word0, *values = nw + nodes;
             uint32_t n0 = 0, v = 0;
             for (int j = 0; j < trees; ++j, t += K) {
                 const int64_t a = e.off[t];
@@ -172,11 +174,13 @@ bool pack_trees(const Trees &e, const Shapes &sh, int K, int max_chunk_trees, Pl
                         }
                     }
                     nw[n0 + (uint32_t)i] = ((unsigned long long)hi << 32) | lo;
-                    if (e.cat_bits)
-                        std::memcpy(&p.cat[((size_t)node0 + n0 + (uint32_t)i) * 4], &e.cat_bits[(size_t)nd * 4], 32);
+                    if (cat)
+                        std::memcpy(&cat[((size_t)node0 + n0 + (uint32_t)i) * 4], &e.cat_bits[(size_t)nd * 4], 32);
                 }
+                for (int32_t i = used; i < count; ++i) nw[n0 + (uint32_t)i] = 0;  // not reached
                 n0 += (uint32_t)count;
             }
+            for (int32_t i = (int32_t)v; i < words - nodes; ++i) values[i] = 0;
             word0 += words;
             node0 += nodes;
         }

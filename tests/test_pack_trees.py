@@ -41,8 +41,12 @@ double leaf_of(const Forest &fo, int64_t t, const uint8_t *row) {
     return fo.value[at];
 }
 
+struct Pack : Packed {
+    std::vector<unsigned long long> words;  // their end is guarded
+};
+
 // the packed walk of class k, as the kernels do it; its leaf values in order
-std::vector<double> packed_walk(const Packed &p, int k, const uint8_t *row) {
+std::vector<double> packed_walk(const Pack &p, int k, const uint8_t *row) {
     std::vector<double> got;
     for (int c = p.chunk_of[k]; c < p.chunk_of[k + 1]; ++c) {
         const Chunk &ch = p.chunk[c];
@@ -68,9 +72,12 @@ std::vector<double> packed_walk(const Packed &p, int k, const uint8_t *row) {
     return got;
 }
 
-bool pack(const Forest &fo, int K, Packed &p) {
+bool pack(const Forest &fo, int K, Pack &p) {
     const Trees e = fo.view();
-    return pack_trees(e, check_trees(e, kF), K, 256, [](int32_t f) { return (uint32_t)f; }, p);
+    const Shapes sh = check_trees(e, kF);
+    if (!chunks_hold(sh)) std::printf("a tree past a chunk\n"), std::exit(1);
+    p.words.resize((size_t)sh.words);
+    return pack_trees(e, sh, K, 256, [](int32_t f) { return (uint32_t)f; }, p.words.data(), nullptr, p);
 }
 
 int main(int argc, char **argv) {
@@ -123,7 +130,7 @@ int main(int argc, char **argv) {
             }
             fo.end();
         }
-        Packed p;
+        Pack p;
         if (!pack(fo, K, p)) {
             if (must_pack) return std::printf("round %d: not packed\n", round), 1;
             ++refused;
@@ -148,14 +155,14 @@ int main(int argc, char **argv) {
         fo.node(0, 3, 3, 4), fo.node(1, 3, 2, 5), fo.node(1, 3, 5, 6), fo.node(1, 3, 5, 6), fo.node(2, 3, 6, 5);
         fo.node(-1, 0, -1, -1), fo.node(-1, 0, -1, -1), fo.end();
         if (more) fo.node(-1, 0, -1, -1), fo.end();
-        Packed p;
+        Pack p;
         if (pack(fo, 1, p)) return std::printf("a node reached twice was packed\n"), 1;
     }
     // one leaf for every split
     Forest fo;
     for (int i = 0; i < 3; ++i) fo.node(0, 3, 3, 3);
     fo.node(-1, 0, -1, -1), fo.end();
-    Packed p;
+    Pack p;
     if (pack(fo, 1, p)) return std::printf("a leaf reached twice was packed\n"), 1;
     return 0;
 }
