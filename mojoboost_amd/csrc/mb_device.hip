@@ -659,6 +659,9 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
             if (c <= mb::kMaxQueryRows) order[(size_t)at[c]++] = (int32_t)q;
         }
         s.n_small = (int32_t)(nq - (int64_t)big.size());
+        // at[c] is now the place behind the queries of c documents
+        s.n_few = s.n_small - at[mb::kRankFew + 1];
+        if (s.n_few < mb::kRankFewLeast) s.n_few = 0;
         int32_t *d_order = dalloc<int32_t>(order.size(), run.arena);
         HIPX(hipMemcpy(d_order, order.data(), order.size() * sizeof(int32_t), hipMemcpyHostToDevice));
         s.rank_order = d_order;

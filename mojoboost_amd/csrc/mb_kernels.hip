@@ -366,30 +366,44 @@ __global__ __launch_bounds__(256) void k_objective(DevState s) {
 // per SIMD; held to 80 or 64 registers for six or eight: 180, 188), 1534
 // with one rank at a time, a branch and a dependent LDS read per pair and the
 // block waiting at two barriers per rank.
+// Many queries of few documents (kRankFewLeast of at most kRankFew) take blocks
+// of two waves instead, eight of them on a CU where two of 512 threads fit:
+// such a query is over in the latency of its sort and barriers, whatever the
+// block, and a 512-thread one costs 6 us of a slot. 100K documents in queries
+// of 1: 804 -> 189 us, of 3: 394 -> 121, of 8: 167 -> 66, of 32: 115 -> 59
+// (219, 215, 215 and 301 with one rank at a time in 256 threads); fewer
+// such queries are not worth a launch beside the large ones' (some 5 us).
 constexpr int kRankThreads = 512;
-constexpr int kRankEval = kRankThreads - 64;  // pairs of a tile, at most, when it has several ranks
+constexpr int kRankFewThreads = 128;
+// pairs of a tile, at most, when it has several ranks: one per evaluating thread
+constexpr int rank_eval(int threads) { return threads - 64; }
 // LDS of queries padded to `pad` documents (a power of two, at least 8): per
 // document the sort key and position, the gain of its label, its discount and
 // its two sums; two tiles of two values per pair; and two blocks of eight
 // values the walk may read past the last tile.
-__host__ __device__ constexpr int rank_tile_pairs(int pad) { return pad > kRankEval ? pad : kRankEval; }
-__host__ __device__ constexpr size_t rank_lds_for(int pad) {
-    return (size_t)pad * 44 + (size_t)rank_tile_pairs(pad) * 32 + 16 * 8;
+__host__ __device__ constexpr int rank_tile_pairs(int threads, int pad) {
+    return pad > threads - 64 ? pad : threads - 64;
 }
-static_assert(rank_lds_for(kMaxQueryRows) + 1024 <= 160 * 1024, "the largest LDS query");
+__host__ __device__ constexpr size_t rank_lds_for(int threads, int pad) {
+    return (size_t)pad * 44 + (size_t)rank_tile_pairs(threads, pad) * 32 + 16 * 8;
+}
+static_assert(rank_lds_for(kRankThreads, kMaxQueryRows) + 1024 <= 160 * 1024, "the largest LDS query");
 __device__ __forceinline__ bool rank_before(double ka, int ia, double kb, int ib) {
     return ka > kb || (ka == kb && ia < ib);
 }
 
-__global__ __launch_bounds__(kRankThreads) void k_lambdarank(DevState s) {
+// Queries [first, end) of rank_order, of at most P documents each.
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void k_lambdarank(DevState s, unsigned first, unsigned end, int P) {
+    constexpr int kEval = rank_eval(kThreads);
     extern __shared__ unsigned char rank_lds[];
     __shared__ double s_factor;
-    __shared__ double red_g[kRankThreads / 64], red_h[kRankThreads / 64];
+    __shared__ double red_g[kThreads / 64], red_h[kThreads / 64];
     const Round rd = *s.round;
     if (rd.stopped) return;
     const HyperParams &hp = s.hp;
     if (blockIdx.x == 0 && threadIdx.x == 0) s.cursor[0] = 0;  // root row count
-    const int P = s.rank_pad, cap = rank_tile_pairs(P);
+    const int cap = rank_tile_pairs(kThreads, P);
     double *key = (double *)rank_lds;
     double *G = key + P;
     double *H = G + P;
@@ -404,7 +418,7 @@ __global__ __launch_bounds__(kRankThreads) void k_lambdarank(DevState s) {
     const uint64_t bstream = hp.bagging ? bag_stream_of(hp, rd.round) : 0;
     const int64_t bfall = hp.bagging ? bag_fallback_of(s, rd.round) : -1;
     double mg = 0.0, mh = 0.0;
-    for (unsigned qi = blockIdx.x; qi < (unsigned)s.n_small; qi += gridDim.x) {
+    for (unsigned qi = first + blockIdx.x; qi < end; qi += gridDim.x) {
         const int q = s.rank_order[qi];
         const int64_t a = s.qstart[q];
         const int cnt = (int)(s.qstart[q + 1] - a);
@@ -446,11 +460,11 @@ __global__ __launch_bounds__(kRankThreads) void k_lambdarank(DevState s) {
         // a rank's row of a tile: its pairs at j, -0.0 at every j <= i and
         // from cnt to the next multiple of eight
         const int row = (cnt + 7) & ~7;
-        const int tile = kRankEval / row > 1 ? kRankEval / row : 1;  // ranks of a tile: tile x row <= cap
+        const int tile = kEval / row > 1 ? kEval / row : 1;  // ranks of a tile: tile x row <= cap
         auto evaluate = [&](int i0, int b) {
             const int rows = top - i0 < tile ? top - i0 : tile;
             double *sg = SG + b * cap, *sh = SH + b * cap;
-            for (int e = tid - 64; e < rows * row; e += kRankEval) {
+            for (int e = tid - 64; e < rows * row; e += kEval) {
                 const int ii = e / row, j = e - ii * row, i = i0 + ii;
                 double vg = -0.0, vh = -0.0;
                 const double gi = gain[i], gj = j < cnt ? gain[j] : gi;
@@ -6255,13 +6269,22 @@ __global__ void k_exp_sigmoid(const double *x, double *e, double *sg, int64_t n)
 }
 
 // ------------------------------------------------------------------ launch
-size_t rank_lds_bytes(const DevState &s) { return rank_lds_for(s.rank_pad); }
+size_t rank_lds_bytes(const DevState &s) { return rank_lds_for(kRankThreads, s.rank_pad); }
 hipError_t launch_objective(const DevState &s, int grid, hipStream_t st) {
     if (s.hp.objective == kObjLambdarank) {
         // a block per query, as many as may be in flight; the next queries
         // of rank_order go to the blocks that end first
-        hipLaunchKernelGGL(k_lambdarank, dim3(launch_blocks(s.n_small, kRankThreads)), dim3(kRankThreads),
-                           rank_lds_bytes(s), st, s);
+        const unsigned split = (unsigned)(s.n_small - s.n_few), end = (unsigned)s.n_small;
+        if (split > 0 || s.n_few == 0)
+            hipLaunchKernelGGL(k_lambdarank<kRankThreads>, dim3(launch_blocks(split, kRankThreads)), dim3(kRankThreads),
+                               rank_lds_bytes(s), st, s, 0u, split, s.rank_pad);
+        if (s.n_few > 0) {
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return e;
+            hipLaunchKernelGGL(k_lambdarank<kRankFewThreads>, dim3(launch_blocks(s.n_few, kRankFewThreads)),
+                               dim3(kRankFewThreads), rank_lds_for(kRankFewThreads, kRankFew), st, s, split, end,
+                               kRankFew);
+        }
         if (s.n_big > 0) {
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
@@ -6352,7 +6375,7 @@ hipError_t planner_fits(const DevState &s, bool *fits) {
 
 hipError_t prepare_kernels(const DevState &s) {
     const size_t h = hist_lds_bytes(s);
-    if (s.hp.objective == kObjLambdarank) MB_SET_LDS(k_lambdarank, rank_lds_bytes(s));
+    if (s.hp.objective == kObjLambdarank) MB_SET_LDS(k_lambdarank<kRankThreads>, rank_lds_bytes(s));
     if (s.hp.stage16) {
         MB_SET_LDS((k_hist<1, WAcc16>), h);
         MB_SET_LDS((k_hist<2, WAcc16>), h);

@@ -17,6 +17,10 @@ constexpr int kObjBinary = 1;
 constexpr int kObjMulticlass = 2;
 constexpr int kObjLambdarank = 3;
 constexpr int kMaxQueryRows = 2048;  // the largest query the LDS sort takes (larger: k_lambdarank_big)
+// Queries of at most kRankFew documents take k_lambdarank's small blocks where
+// there are kRankFewLeast of them.
+constexpr int kRankFew = 32;  // a power of two, as the LDS is laid out
+constexpr int kRankFewLeast = 2048;
 
 // Leaf-wise growth, batched. The reference grows a tree best-first: split the
 // frontier leaf of largest gain, score both children, repeat. A leaf's best
@@ -321,6 +325,7 @@ struct DevState {
     int32_t n_queries;
     int32_t n_small;                // queries of at most kMaxQueryRows rows
     const int32_t *rank_order;      // n_small: those queries, largest first
+    int32_t n_few;                  // the last of rank_order, of at most kRankFew rows, for the small blocks (0: none)
     int32_t rank_pad;               // largest query of at most kMaxQueryRows rows, rounded up to a power of two (at least 8)
     // queries of more than kMaxQueryRows rows (k_lambdarank_big): their
     // indices, and per block slot the query's keys, G, H (binary64) and
