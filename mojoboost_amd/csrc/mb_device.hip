@@ -505,6 +505,7 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
     const int max_nodes = 2 * L - 1;
     const int F = ds->F;
     mb::DevState &s = tb.s;
+    mb::ZeroList zero;
     const bool quantized = p->use_quantized_grad != 0;
     const bool wide = quantized && p->quant_scale_rule == 1;
     const bool stage16 = wide && p->quant_staging == 1;
@@ -546,7 +547,7 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
         if (!stage16) s.gq = dalloc<int32_t>(2 * (size_t)ds->n, run.arena);
         s.magpart = dalloc<float>(2 * 256, run.arena);
         s.stage16_over = dalloc<unsigned long long>(2, run.arena);
-        HIPX(hipMemset(s.stage16_over, 0, 2 * sizeof(unsigned long long)));
+        zero.add(s.stage16_over, 2 * sizeof(unsigned long long));
     }
     s.enodes = dalloc<mb::ENode>(s.e_cap, run.arena);
     s.items = dalloc<mb::Item>(s.kmax, run.arena);
@@ -582,8 +583,8 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
         s.e_cat = dalloc<unsigned long long>((size_t)s.e_cap * 4, run.arena);
         s.t_cat = dalloc<unsigned long long>((size_t)max_nodes * 4, run.arena);
         s.arc_cat = dalloc<unsigned long long>((size_t)T * max_nodes * 4, run.arena);
-        HIPX(hipMemset(s.t_cat, 0, (size_t)max_nodes * 4 * sizeof(unsigned long long)));
-        HIPX(hipMemset(s.arc_cat, 0, (size_t)T * max_nodes * 4 * sizeof(unsigned long long)));
+        zero.add(s.t_cat, (size_t)max_nodes * 4 * sizeof(unsigned long long));
+        zero.add(s.arc_cat, (size_t)T * max_nodes * 4 * sizeof(unsigned long long));
     }
     s.max_nodes = max_nodes;
     uint8_t *fmask = dalloc<uint8_t>((size_t)T * F, run.arena);
@@ -612,7 +613,7 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
         s.grad64 = dalloc<double>(ds->n, run.arena);
         s.hess64 = dalloc<double>(ds->n, run.arena);
         s.stats64 = dalloc<unsigned long long>(4, run.arena);
-        HIPX(hipMemset(s.stats64, 0, 4 * sizeof(unsigned long long)));
+        zero.add(s.stats64, 4 * sizeof(unsigned long long));
         const int64_t nq = (int64_t)ds->qstart.size() - 1;
         std::vector<double> disc(ds->max_query), inv(nq);
         for (int i = 0; i < ds->max_query; ++i) disc[i] = 1.0 / mb::ref_log2((double)i + 2.0);
@@ -718,10 +719,10 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
         s.goss_urow = dalloc<int32_t>(ds->n, run.arena);
         s.goss_umask = dalloc<unsigned long long>((ds->n + 63) / 64, run.arena);
         s.goss_other = dalloc<uint8_t>(ds->n, run.arena);
-        HIPX(hipMemset(s.goss_other, 0, ds->n));
+        zero.add(s.goss_other, ds->n);
         s.goss_rows = dalloc<int32_t>(ds->n, run.arena);
         s.goss_max = dalloc<unsigned long long>(4, run.arena);
-        HIPX(hipMemset(s.goss_max, 0, 4 * sizeof(unsigned long long)));
+        zero.add(s.goss_max, 4 * sizeof(unsigned long long));
         if (p->objective == MBH_OBJ_MULTICLASS) s.goss_imp = dalloc<double>(ds->n, run.arena);
     }
     hp.bagging = (p->bagging_freq > 0 && p->bagging_fraction < 1.0) ? 1 : 0;
@@ -785,18 +786,19 @@ TrainBuffers setup_state(mbh_dataset *ds, const mbh_params *p, Run &run, int64_t
     if (!mb::plan_fits(L, mb::plan_lds_bytes(s), 0)) refuse_planner();
     if (mb::hist_lds_bytes(s) + kPbStaticLds > 160 * 1024)
         throw Error{MOJOTREES_ERROR_TRAINING, "internal: the feature tile exceeds one workgroup's LDS"};
-    HIPX(hipMemset(s.rows0, 0, (size_t)ds->n * sizeof(int32_t)));
-    HIPX(hipMemset(s.rows1, 0, (size_t)ds->n * sizeof(int32_t)));
-    HIPX(hipMemset(s.stats, 0, 4 * mb::kStatSlots * sizeof(uint32_t)));
-    HIPX(hipMemset(s.batch, 0, sizeof(mb::Batch)));
-    HIPX(hipMemset(s.grow, 0, sizeof(mb::Grow)));
-    HIPX(hipMemset(s.part_items, 0, (size_t)s.kmax * sizeof(mb::PartItem)));
-    HIPX(hipMemset(s.acc_items, 0, (size_t)s.kmax * sizeof(mb::AccItem)));
-    HIPX(hipMemset(s.cursor, 0, (2 + 2 * (size_t)s.kmax) * sizeof(int64_t)));
-    HIPX(hipMemset(s.error, 0, sizeof(int32_t)));
-    HIPX(hipMemset(s.t_meta, 0, 2 * sizeof(int32_t)));
-    HIPX(hipMemset(s.arc_aux, 0, (size_t)T * 4 * sizeof(int64_t)));
-    HIPX(hipMemset(s.arc_int, 0, (size_t)T * (6 * max_nodes + 2) * sizeof(int32_t)));
+    zero.add(s.rows0, (size_t)ds->n * sizeof(int32_t));
+    zero.add(s.rows1, (size_t)ds->n * sizeof(int32_t));
+    zero.add(s.stats, 4 * mb::kStatSlots * sizeof(uint32_t));
+    zero.add(s.batch, sizeof(mb::Batch));
+    zero.add(s.grow, sizeof(mb::Grow));
+    zero.add(s.part_items, (size_t)s.kmax * sizeof(mb::PartItem));
+    zero.add(s.acc_items, (size_t)s.kmax * sizeof(mb::AccItem));
+    zero.add(s.cursor, (2 + 2 * (size_t)s.kmax) * sizeof(int64_t));
+    zero.add(s.error, sizeof(int32_t));
+    zero.add(s.t_meta, 2 * sizeof(int32_t));
+    zero.add(s.arc_aux, (size_t)T * 4 * sizeof(int64_t));
+    zero.add(s.arc_int, (size_t)T * (6 * max_nodes + 2) * sizeof(int32_t));
+    HIPX(mb::launch_zero(zero, ds->n_cu, nullptr));
     mb::Round r0 = mb::initial_round();
     HIPX(hipMemcpy(s.round, &r0, sizeof(r0), hipMemcpyHostToDevice));
     std::vector<uint8_t> masks((size_t)T * F);
@@ -862,6 +864,7 @@ mb::DevState clone_class_state(const mb::DevState &s0, const mbh_dataset *ds, in
     const int F = ds->F;
     s.hp.class_stride = stride;
     const size_t rec_total = (size_t)s0.n_tiles * (size_t)n * (size_t)s0.rec_bytes;
+    mb::ZeroList zero;
     uint8_t *rec = dalloc<uint8_t>(rec_total, run.arena);
     HIPX(hipMemcpy(rec, s0.records, rec_total, hipMemcpyDeviceToDevice));
     s.records = rec;
@@ -885,11 +888,11 @@ mb::DevState clone_class_state(const mb::DevState &s0, const mbh_dataset *ds, in
     if (s0.magpart) s.magpart = dalloc<float>(2 * 256, run.arena);
     if (s0.stage16_over) {
         s.stage16_over = dalloc<unsigned long long>(2, run.arena);
-        HIPX(hipMemset(s.stage16_over, 0, 2 * sizeof(unsigned long long)));
+        zero.add(s.stage16_over, 2 * sizeof(unsigned long long));
     }
     if (s0.goss_max) {
         s.goss_max = dalloc<unsigned long long>(4, run.arena);
-        HIPX(hipMemset(s.goss_max, 0, 4 * sizeof(unsigned long long)));
+        zero.add(s.goss_max, 4 * sizeof(unsigned long long));
     }
     s.enodes = dalloc<mb::ENode>(s.e_cap, run.arena);
     s.items = dalloc<mb::Item>(s.kmax, run.arena);
@@ -920,17 +923,18 @@ mb::DevState clone_class_state(const mb::DevState &s0, const mbh_dataset *ds, in
         s.scan_cat = dalloc<unsigned long long>((size_t)s.kmax * 2 * F * 4, run.arena);
         s.e_cat = dalloc<unsigned long long>((size_t)s.e_cap * 4, run.arena);
         s.t_cat = dalloc<unsigned long long>((size_t)max_nodes * 4, run.arena);
-        HIPX(hipMemset(s.t_cat, 0, (size_t)max_nodes * 4 * sizeof(unsigned long long)));
+        zero.add(s.t_cat, (size_t)max_nodes * 4 * sizeof(unsigned long long));
     }
-    HIPX(hipMemset(s.rows0, 0, (size_t)n * sizeof(int32_t)));
-    HIPX(hipMemset(s.rows1, 0, (size_t)n * sizeof(int32_t)));
-    HIPX(hipMemset(s.stats, 0, 4 * mb::kStatSlots * sizeof(uint32_t)));
-    HIPX(hipMemset(s.batch, 0, sizeof(mb::Batch)));
-    HIPX(hipMemset(s.grow, 0, sizeof(mb::Grow)));
-    HIPX(hipMemset(s.part_items, 0, (size_t)s.kmax * sizeof(mb::PartItem)));
-    HIPX(hipMemset(s.acc_items, 0, (size_t)s.kmax * sizeof(mb::AccItem)));
-    HIPX(hipMemset(s.cursor, 0, (2 + 2 * (size_t)s.kmax) * sizeof(int64_t)));
-    HIPX(hipMemset(s.t_meta, 0, 2 * sizeof(int32_t)));
+    zero.add(s.rows0, (size_t)n * sizeof(int32_t));
+    zero.add(s.rows1, (size_t)n * sizeof(int32_t));
+    zero.add(s.stats, 4 * mb::kStatSlots * sizeof(uint32_t));
+    zero.add(s.batch, sizeof(mb::Batch));
+    zero.add(s.grow, sizeof(mb::Grow));
+    zero.add(s.part_items, (size_t)s.kmax * sizeof(mb::PartItem));
+    zero.add(s.acc_items, (size_t)s.kmax * sizeof(mb::AccItem));
+    zero.add(s.cursor, (2 + 2 * (size_t)s.kmax) * sizeof(int64_t));
+    zero.add(s.t_meta, 2 * sizeof(int32_t));
+    HIPX(mb::launch_zero(zero, ds->n_cu, nullptr));
     mb::Round r0 = mb::initial_round();
     r0.class_k = first;
     r0.tree_index = first;

@@ -60,6 +60,23 @@ hipError_t launch_build_records(const uint8_t *bins_cm, uint8_t *records, int64_
                                 int tile_f, int n_tiles, int grid, hipStream_t st);
 // n x K row-major from class-major scores.
 hipError_t launch_row_major(const double *in, double *out, int64_t n, int K, hipStream_t st);
+// Buffers of an arena (aligned, and padded to 256 bytes) that a call's start
+// zeroes, in one launch: a hipMemset each took 12 us of the host in a slab,
+// 12 of them a call.
+struct ZeroList {
+    static constexpr int kMost = 24;
+    uint4 *p[kMost];
+    uint64_t words[kMost];  // of 16 bytes
+    int n = 0;
+    void add(void *at, size_t bytes) {
+        if (n < kMost) {
+            p[n] = (uint4 *)at;
+            words[n] = (bytes + 15) / 16;
+        }
+        ++n;  // past kMost: the launch is refused
+    }
+};
+hipError_t launch_zero(const ZeroList &z, int n_cu, hipStream_t st);
 hipError_t launch_fill_f64(double *p, int64_t n, int K, const double *base, int grid, hipStream_t st);
 hipError_t launch_exp_sigmoid(const double *x, double *e, double *sg, int64_t n, hipStream_t st);
 

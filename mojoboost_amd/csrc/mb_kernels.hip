@@ -6260,6 +6260,13 @@ __global__ __launch_bounds__(256) void k_fill_f64(double *p, int64_t n, int K, c
         p[i] = base[i / n];
 }
 
+__global__ __launch_bounds__(256) void k_zero(ZeroList z) {
+    const uint64_t stride = (uint64_t)gridDim.x * 256;
+    for (int i = 0; i < z.n; ++i)
+        for (uint64_t w = (uint64_t)blockIdx.x * 256 + threadIdx.x; w < z.words[i]; w += stride)
+            z.p[i][w] = make_uint4(0u, 0u, 0u, 0u);
+}
+
 __global__ void k_exp_sigmoid(const double *x, double *e, double *sg, int64_t n) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) {
@@ -6592,6 +6599,14 @@ hipError_t launch_row_major(const double *in, double *out, int64_t n, int K, hip
     const unsigned grid = (unsigned)std::min<int64_t>((n + 63) / 64, kRowMajorBlocks);
     hipLaunchKernelGGL(k_row_major, dim3(grid, (unsigned)((K + kRowMajorK - 1) / kRowMajorK)), dim3(256), 0, st, in,
                        out, n, K);
+    return hipGetLastError();
+}
+hipError_t launch_zero(const ZeroList &z, int n_cu, hipStream_t st) {
+    if (z.n > ZeroList::kMost) return hipErrorInvalidValue;
+    uint64_t most = 1;
+    for (int i = 0; i < z.n; ++i) most = std::max(most, z.words[i]);
+    const unsigned grid = (unsigned)std::min<uint64_t>((most + 255) / 256, 8 * (uint64_t)n_cu);
+    hipLaunchKernelGGL(k_zero, dim3(grid), dim3(256), 0, st, z);
     return hipGetLastError();
 }
 hipError_t launch_fill_f64(double *p, int64_t n, int K, const double *base, int grid, hipStream_t st) {
