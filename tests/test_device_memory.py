@@ -121,6 +121,13 @@ int main() {
     }
     slab_pool().drop(&a);
     CHECK(card.used == 0 && card.live.empty());
+
+    // a call on no dataset takes what it places, and leaves nothing
+    {
+        Arena run(nullptr);
+        CHECK(place(run, 1000) && place(run, 1000) && card.used == 2048);
+    }
+    CHECK(card.used == 0);
     return 0;
 }
 """
