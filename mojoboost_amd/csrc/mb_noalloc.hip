@@ -41,7 +41,11 @@ constexpr int kTargetBlocks = 1024;
 constexpr int kMinChunk = 1024;
 constexpr int kOldMinChunk = 2048;     // rows per chunk behind the size limit's wording (below)
 constexpr int kMergeThreads = 256;
-constexpr int kMergeCells = 32;        // cells of a merge block, kMergeThreads / kMergeCells threads each
+// Cells of a merge block, of kMergeThreads / kMergeCells threads each.
+constexpr int kMergeCells = 32;
+// From this many cells on, fewer partials than those threads are summed by a
+// thread a cell (k_na_merge has both sides' figures).
+constexpr int kMergeMany = 1 << 16;
 
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -167,17 +171,21 @@ __global__ __launch_bounds__(kThreads) void k_na_hist(const uint8_t *__restrict_
     for (int i = threadIdx.x; i < nf * nb; i += kThreads) out[i] = lds[i];
 }
 
-// kMergeCells (feature, bin) cells per block, each summed by several threads
-// (thread t takes the partials t / kMergeCells, + threads per cell, ..., four
+// kCells (feature, bin) cells per block, each summed by several threads
+// (thread t takes the partials t / kCells, + threads per cell, ..., four
 // loads in flight), then over LDS: int32 {grad, hess, count}. One thread per
 // cell walked every partial alone, 28 blocks in all for 28 x 255 cells
-// (68 us; 5 us this way).
+// (68 us; 5 us this way). Where the cells alone fill the chip and the
+// partials are fewer than the threads, most of which would idle, a thread a
+// cell: 2.05M cells, 1 partial: 25.7 -> 8.6 us; 1.02M, 2: 14.2 -> 7.0; 510K,
+// 4: 8.4 -> 5.8 (7.7K cells, 6 partials: 2.3 against 3.2 us).
+template <int kCells>
 __global__ __launch_bounds__(kMergeThreads) void k_na_merge(const unsigned long long *__restrict__ part, int blocks,
                                                            int cells, int32_t *__restrict__ out) {
-    constexpr int kPer = kMergeThreads / kMergeCells;
-    __shared__ int sum[3][kPer][kMergeCells];
-    const int lc = threadIdx.x % kMergeCells, p = threadIdx.x / kMergeCells;
-    const int c = (int)blockIdx.x * kMergeCells + lc;
+    constexpr int kPer = kMergeThreads / kCells;
+    __shared__ int sum[3][kPer][kCells];
+    const int lc = threadIdx.x % kCells, p = threadIdx.x / kCells;
+    const int c = (int)blockIdx.x * kCells + lc;
     // int32 sums: the caller's rows x (B + 1) stay below 2^31
     int g = 0, h = 0, cnt = 0;
     auto add = [&](unsigned long long v) {
@@ -200,13 +208,13 @@ __global__ __launch_bounds__(kMergeThreads) void k_na_merge(const unsigned long 
     sum[1][p][lc] = h;
     sum[2][p][lc] = cnt;
     __syncthreads();
-    // the block's 3 x kMergeCells outputs, consecutive in memory
-    for (int i = threadIdx.x; i < 3 * kMergeCells; i += kMergeThreads) {
+    // the block's 3 x kCells outputs, consecutive in memory
+    for (int i = threadIdx.x; i < 3 * kCells; i += kMergeThreads) {
         const int cell = i / 3, k = i - 3 * cell;
-        if ((int)blockIdx.x * kMergeCells + cell >= cells) break;
+        if ((int)blockIdx.x * kCells + cell >= cells) break;
         int v = 0;
         for (int q = 0; q < kPer; ++q) v += sum[k][q][cell];
-        out[(size_t)3 * blockIdx.x * kMergeCells + i] = v;
+        out[(size_t)3 * blockIdx.x * kCells + i] = v;
     }
 }
 
@@ -281,8 +289,11 @@ extern "C" int32_t mbh_histogram_noalloc(const uint8_t *bins_cm, int64_t n_rows,
                        dim3(kThreads), (size_t)ft * n_bins * sizeof(unsigned long long), st, bins_cm, n_rows,
                        (int)n_features, (int)n_bins, q_grad, q_hess, rows, m, chunk, ft, B / 2 + 1, B + 1, part,
                        status);
-    hipLaunchKernelGGL(k_na_merge, dim3((unsigned)((cells + kMergeCells - 1) / kMergeCells)), dim3(kMergeThreads), 0,
-                       st, (const unsigned long long *)part, (int)blocks, cells, out);
+    const bool single = cells >= kMergeMany && blocks < kMergeThreads / kMergeCells;
+    const int mc = single ? kMergeThreads : kMergeCells;
+    hipLaunchKernelGGL(single ? k_na_merge<kMergeThreads> : k_na_merge<kMergeCells>,
+                       dim3((unsigned)((cells + mc - 1) / mc)), dim3(kMergeThreads), 0, st,
+                       (const unsigned long long *)part, (int)blocks, cells, out);
     e = hipGetLastError();
     if (e != hipSuccess) {
         set_err(err, err_len, hipGetErrorString(e));

@@ -26,6 +26,10 @@ def _want(bins, qg, qh, rows, f, nb):
     (300_000, 3, 7, 299_999),    # the hottest bins
     (1_200_000, 28, 255, None),  # chunks above the smallest
     (200, 9_000, 2, 150),        # more than kMaxTiles x kTileFeatures features
+    (40, 256, 256, None),        # the first cells merged by a thread each, one partial
+    (3_000, 2_100, 255, 2_500),  # three partials, a ragged last merge block
+    (9_000, 255, 256, None),     # just below them
+    (40_000, 300, 255, None),    # eight partials, a cell's threads each one
 ])
 def test_noalloc_shapes(n, f, nb, sel):
     rng = np.random.default_rng(n + f)
