@@ -55,6 +55,13 @@ constexpr int kMinRows = 4;      // rows of a block, at least
 // split until about as many blocks of k_predict_wide share the work (each
 // stages every tree of its class once, so not more).
 constexpr int kBlocksTarget = 512;
+// Of a matrix in several batches, columns of at least kLongColumn rows are
+// copied each on its own, shorter ones gathered kStageBytes at a time: a copy
+// costs some 9 us beside its bytes. 200K rows x 20,000 (columns of 107K and
+// 93K) 441 ms on their own, 213 gathered; 24K x 100,000 1900 and 141; 2.2M x
+// 1,000 89 and 150.
+constexpr int64_t kLongColumn = 1 << 18;
+constexpr int64_t kStageBytes = (int64_t)16 << 20;
 
 struct PredictArgs {
     const uint8_t *bins;  // F x n, column-major
@@ -398,13 +405,26 @@ extern "C" int32_t mbh_predict_binned(const uint8_t *bins_cm, int64_t n, int32_t
         const Kernel kernel = pick_kernel(rows, lds_bins, p.missing, cat_bits != nullptr);
         if (packed)
             HIPP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        std::unique_ptr<uint8_t[]> stage;
         for (int64_t r0 = 0; r0 < n; r0 += batch) {
             const int64_t m = std::min(batch, n - r0);
             a.n = m;
             // one batch is the caller's matrix as it lies; of several, each
             // column's part
-            if (m == n) HIPP(hipMemcpyAsync(d.p + at_bins, bins_cm, (size_t)F * m, hipMemcpyHostToDevice, 0));
-            else HIPP(hipMemcpy2DAsync(d.p + at_bins, m, bins_cm + r0, n, m, F, hipMemcpyHostToDevice, 0));
+            if (m == n) {
+                HIPP(hipMemcpyAsync(d.p + at_bins, bins_cm, (size_t)F * m, hipMemcpyHostToDevice, 0));
+            } else if (m >= kLongColumn) {
+                HIPP(hipMemcpy2DAsync(d.p + at_bins, m, bins_cm + r0, n, m, F, hipMemcpyHostToDevice, 0));
+            } else {
+                const int64_t cols = std::max<int64_t>(1, std::min<int64_t>(F, kStageBytes / m));
+                if (!stage) stage.reset(new uint8_t[(size_t)std::max<int64_t>(kStageBytes, m)]);
+                for (int64_t f0 = 0; f0 < F; f0 += cols) {
+                    const int64_t nf = std::min<int64_t>(cols, F - f0);
+                    for (int64_t f = 0; f < nf; ++f)
+                        std::memcpy(stage.get() + f * m, bins_cm + (size_t)(f0 + f) * n + r0, (size_t)m);
+                    HIPP(hipMemcpy(d.p + at_bins + (size_t)f0 * m, stage.get(), (size_t)(nf * m), hipMemcpyHostToDevice));
+                }
+            }
             if (!packed) {
                 const int grid = (int)std::min<int64_t>((m + 255) / 256, 4096);
                 hipLaunchKernelGGL(k_predict, dim3(grid, K), dim3(256), 0, 0, a);
