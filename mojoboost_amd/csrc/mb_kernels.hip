@@ -392,9 +392,8 @@ __device__ __forceinline__ bool rank_before(double ka, int ia, double kb, int ib
     return ka > kb || (ka == kb && ia < ib);
 }
 
-// Queries [first, end) of rank_order, of at most P documents each.
 template <int kThreads>
-__global__ __launch_bounds__(kThreads) void k_lambdarank(DevState s, unsigned first, unsigned end, int P) {
+__global__ __launch_bounds__(kThreads) void k_lambdarank(DevState s) {
     constexpr int kEval = rank_eval(kThreads);
     extern __shared__ unsigned char rank_lds[];
     __shared__ double s_factor;
@@ -403,7 +402,7 @@ __global__ __launch_bounds__(kThreads) void k_lambdarank(DevState s, unsigned fi
     if (rd.stopped) return;
     const HyperParams &hp = s.hp;
     if (blockIdx.x == 0 && threadIdx.x == 0) s.cursor[0] = 0;  // root row count
-    const int cap = rank_tile_pairs(kThreads, P);
+    const int P = s.rank_pad, cap = rank_tile_pairs(kThreads, P);
     double *key = (double *)rank_lds;
     double *G = key + P;
     double *H = G + P;
@@ -418,7 +417,7 @@ __global__ __launch_bounds__(kThreads) void k_lambdarank(DevState s, unsigned fi
     const uint64_t bstream = hp.bagging ? bag_stream_of(hp, rd.round) : 0;
     const int64_t bfall = hp.bagging ? bag_fallback_of(s, rd.round) : -1;
     double mg = 0.0, mh = 0.0;
-    for (unsigned qi = first + blockIdx.x; qi < end; qi += gridDim.x) {
+    for (int qi = blockIdx.x; (unsigned)qi < (unsigned)s.n_small; qi += gridDim.x) {
         const int q = s.rank_order[qi];
         const int64_t a = s.qstart[q];
         const int cnt = (int)(s.qstart[q + 1] - a);
@@ -6281,16 +6280,22 @@ hipError_t launch_objective(const DevState &s, int grid, hipStream_t st) {
     if (s.hp.objective == kObjLambdarank) {
         // a block per query, as many as may be in flight; the next queries
         // of rank_order go to the blocks that end first
-        const unsigned split = (unsigned)(s.n_small - s.n_few), end = (unsigned)s.n_small;
-        if (split > 0 || s.n_few == 0)
+        const int split = s.n_small - s.n_few;
+        if (split > 0 || s.n_few == 0) {
+            DevState large = s;
+            large.n_small = split;
             hipLaunchKernelGGL(k_lambdarank<kRankThreads>, dim3(launch_blocks(split, kRankThreads)), dim3(kRankThreads),
-                               rank_lds_bytes(s), st, s, 0u, split, s.rank_pad);
+                               rank_lds_bytes(s), st, large);
+        }
         if (s.n_few > 0) {
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return e;
+            DevState few = s;
+            few.rank_order += split;
+            few.n_small = s.n_few;
+            few.rank_pad = kRankFew;
             hipLaunchKernelGGL(k_lambdarank<kRankFewThreads>, dim3(launch_blocks(s.n_few, kRankFewThreads)),
-                               dim3(kRankFewThreads), rank_lds_for(kRankFewThreads, kRankFew), st, s, split, end,
-                               kRankFew);
+                               dim3(kRankFewThreads), rank_lds_for(kRankFewThreads, kRankFew), st, few);
         }
         if (s.n_big > 0) {
             const hipError_t e = hipGetLastError();
