@@ -24,8 +24,9 @@
 // for 501 rows): 1M rows x 200 trees of 255 leaves 6525 us, now 1080;
 // 501 rows x 100 trees of 31 leaves 488 us, now 27.
 //
-// Trees of more words than a chunk (files may hold them) and more features
-// than a word names take k_predict, the plain walk over global memory.
+// Trees of more words than a chunk, trees that reach a node twice (files may
+// hold both) and more features than a word names take k_predict, the plain walk
+// over global memory.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
